@@ -241,9 +241,9 @@ int32_t nhip_matmul_cq_dev(const nhip_weights* w, const int8_t* d_values, const 
  * Q, K, V and Gate projections), each job j computing all of its rows into
  * d_y[j] with row stride ldy[j] (>= its rows), as nhip_matmul_i8_dev
  * (literal: d_scales [tokens], d_offsets and stride unused) or
- * nhip_matmul_cq_dev (codebook) would.  Decode sizes (literal up to 16
- * tokens, codebook up to 4) run as one launch over every job's row tiles;
- * other token counts run the jobs in turn.  Bit-identical with the
+ * nhip_matmul_cq_dev (codebook) would.  Literal batches of up to 16 tokens
+ * and codebook batches of any count run as one launch over every job's row
+ * tiles; literal ones past 16 run the jobs in turn.  Bit-identical with the
  * single-matrix calls.  w and d_y / ldy are host arrays of `count` entries. */
 int32_t nhip_matmul_batch_dev(const nhip_weights* const* w, int32_t count, const int8_t* d_q,
                               const float* d_scales, const float* d_offsets, int32_t stride,

@@ -102,6 +102,28 @@ namespace nhip {
 // order (bit-identical with the decode kernels), else the fused epilogue.
 int32_t launch_gemm_i8(const DeviceWeights* w, const int8_t* q, const float* qscale, int32_t tokens, float* y,
                        int32_t ldy, int32_t row_start, int32_t row_end, bool exact, hipStream_t stream);
+// Prefill matmul of the codebook formats (gemm_cq.hip), more than 16 tokens:
+// 1 to 4 matrices ("jobs") of one format and K over the same activations.  A
+// job's rows [row_start, row_end) of the matrix go to y[t * ldy + n - row0].
+constexpr int kMaxTileJobs = 4;
+struct TileJob {
+    const uint8_t* tiles;
+    const uint16_t* norms;
+    float* y;
+    int32_t ldy, row0, row_start, row_end, tile_begin;
+    float byte_scale;
+    uint32_t table[4];  // Cq2: the codebook bytes; Cq4: the split tables of lut4x
+};
+struct TileMatmul {
+    const int8_t* q;       // [tokens][cols]
+    const float* scales;   // [tokens][stride]
+    const float* offsets;  // [tokens][stride]
+    int32_t tokens, cols, groups, blocks, groups_pad8, stride;
+    int32_t count;
+    int32_t first[kMaxTileJobs + 1];  // the jobs' first row tiles, in job order
+    TileJob job[kMaxTileJobs];
+};
+int32_t launch_gemm_cq(WeightFormat fmt, const TileMatmul& p, bool special, hipStream_t stream);
 // Ragged decode attention (attention_decode.hip); with d_q_out the output
 // rows are also quantized (QuantizeInt8 per row), which needs max_chunks 1
 // and every head in one block.
@@ -287,8 +309,10 @@ int32_t needle3_attention_inputs_impl(const float* d_raw, int32_t rows, int32_t 
 // a quantized output needs every head in one workgroup.
 int decode_attention_lmax(int capacity, int max_chunks);
 int decode_attention_kv_per_block(int group, int kv_heads, int lmax);
-// Token count from which literal int8 matmuls use the prefill kernel.
-constexpr int32_t kGemmMinTokens = 32;
+// Token count from which literal int8 matmuls use the prefill kernel: 20 x 1024
+// x 3072 takes 4.5 us there and 4.7 in the general kernel, 20 x 2048 x 8192 7.5
+// and 22.7, 20 x 4096 x 96 10.8 and 14.5.
+constexpr int32_t kGemmMinTokens = 17;
 }  // namespace nhip
 
 namespace nhip {

@@ -1731,6 +1731,59 @@ bool plan_general_cq(const DeviceWeights* w, MatmulParams& p, int waves, size_t*
     return *lds <= kMaxLds;
 }
 
+// Whether gemm_cq.hip takes a codebook matmul of `tokens` rows over `tiles` row
+// tiles, or the general kernel, whose waves split the groups of a 16 x 16 block
+// while gemm_cq's run through all of them.  The general kernel takes about
+// 3.2 us (Cq4) or 6 us (Cq2, half as many waves busy per block) and 0.3 ns per
+// (block, group); gemm_cq 1.8 us and 0.42 us per group of its chain, and 0.1 ns.
+// Cq4 64 x 2048 x 2048: 5.5 us general, 8.6 here; 256 x 1024 x 2048: 8.3, 7.2;
+// Cq2 128 x 4096 x 768: 11.1, 13.5; 61 x 768 x 1568: 10.5, 4.3.
+bool takes_gemm_cq(WeightFormat fmt, int32_t groups, const int8_t* q, int32_t tokens, int32_t tiles)
+{
+    if (tokens <= 16 || (reinterpret_cast<uintptr_t>(q) & 15)) return false;  // (16-byte copies into LDS)
+    const int64_t blocks = (int64_t)tiles * ((tokens + 15) / 16);
+    return fmt == WeightFormat::Cq4 ? blocks * groups >= 2100 * (int64_t)groups - 7000
+                                    : blocks * groups >= 1333 * (int64_t)groups - 14000;
+}
+
+TileJob tile_job(const DeviceWeights* w, float* y, int32_t ldy, int32_t row_start, int32_t row_end)
+{
+    TileJob j{};
+    j.tiles = w->tiles;
+    j.norms = w->norms;
+    j.y = y;
+    j.ldy = ldy;
+    j.row_start = row_start;
+    j.row_end = row_end;
+    j.tile_begin = row_start / 16;
+    j.byte_scale = w->byte_scale;
+    std::memcpy(j.table, w->format == WeightFormat::Cq4 ? w->split_table : w->table, sizeof(j.table));
+    return j;
+}
+
+TileMatmul tile_matmul(const DeviceWeights* w, const int8_t* q, const float* scales, const float* offsets,
+                       int32_t stride, int32_t tokens)
+{
+    TileMatmul p{};
+    p.q = q;
+    p.scales = scales;
+    p.offsets = offsets;
+    p.tokens = tokens;
+    p.cols = w->cols;
+    p.groups = w->groups;
+    p.blocks = w->blocks;
+    p.groups_pad8 = w->groups_pad8;
+    p.stride = stride;
+    return p;
+}
+
+void add_job(TileMatmul& p, const TileJob& j)
+{
+    p.job[p.count] = j;
+    p.first[p.count + 1] = p.first[p.count] + (j.row_end + 15) / 16 - j.tile_begin;
+    p.count++;
+}
+
 int32_t run_matmul(const DeviceWeights* w, const int8_t* q, const float* scales, const float* offsets,
                    int32_t stride, int32_t tokens, float* y, int32_t ldy, int32_t row_start,
                    int32_t row_end, int32_t* dots, hipStream_t stream)
@@ -1753,6 +1806,11 @@ int32_t run_matmul(const DeviceWeights* w, const int8_t* q, const float* scales,
     const int tiles = p.tile_end - p.tile_begin;
     const int waves = general_waves(tiles, tokens);
     const int m = std::min(16, tokens);
+    if (cq && !dots && takes_gemm_cq(w->format, w->groups, q, tokens, tiles)) {
+        TileMatmul t = tile_matmul(w, q, scales, offsets, stride, tokens);
+        add_job(t, tile_job(w, y, ldy, row_start, row_end));
+        return launch_gemm_cq(w->format, t, w->special_scales != 0, stream);
+    }
     if (w->format == WeightFormat::Int8G32) {
         if (!dots && tokens >= kGemmMinTokens)
             return launch_gemm_i8(w, q, scales, tokens, y, ldy, row_start, row_end, true, stream);
@@ -1926,6 +1984,11 @@ int32_t run_matmul_batch(const DeviceWeights* const* w, int32_t count, const int
                                                       : launch_dec_batch_ti<8, false>(b, waves, lds, stream));
         return w[0]->format == WeightFormat::Cq4 ? launch_cq_batch_gpw<kCq4>(b, gpw, exact, waves, lds, stream)
                                                  : launch_cq_batch_gpw<kCq2>(b, gpw, exact, waves, lds, stream);
+    }
+    if (cq && takes_gemm_cq(w[0]->format, w[0]->groups, q, tokens, b.first[count])) {
+        TileMatmul t = tile_matmul(w[0], q, scales, offsets, stride, tokens);
+        for (int j = 0; j < count; j++) add_job(t, tile_job(w[j], y[j], ldy[j], 0, w[j]->rows));
+        return launch_gemm_cq(w[0]->format, t, exact, stream);
     }
     if (cq) {  // the general kernel over every job's tiles, one launch
         const int waves2 = general_waves(b.first[count], tokens);
