@@ -1,8 +1,8 @@
 // gemm.hip -- prefill matmul of the literal int8 format (many tokens) on
 // gfx950.
 //
-// y[t][n] for a block of 64 tokens x 128 weight rows per workgroup; each of
-// the four waves owns 32 rows (two 16-row weight tiles) and all 64 tokens.
+// y[t][n] for a block of 16 * TI tokens x 64 * TPW weight rows per workgroup;
+// each of the four waves owns TPW 16-row weight tiles and all the tokens.
 // Per 32-element group one v_mfma_i32_16x16x32_i8 per (16-token subtile,
 // 16-row tile) gives the exact int32 group sums D_g (Scalar.cs:162-184);
 // lane l then holds D_g for row l%16 and tokens 4*(l/16)..+3 of the
@@ -23,7 +23,7 @@
 // Weights are the same re-tiled 1 KB blocks as the decode kernels (one
 // dwordx4 per lane is the B operand of two groups), loaded by each wave for
 // its own tiles.  Activations go through LDS: per stage of 4 blocks (256 K
-// elements) 64 tokens x 256 bytes are copied straight from memory into LDS
+// elements) 256 bytes of every token are copied straight from memory into LDS
 // (global_load_lds, 16 bytes per lane, no registers) in an order in which
 // every MFMA A operand is one conflict-free ds_read_b64.  The LDS stage is
 // double-buffered: the next stage's activations, weights and scales are
@@ -41,12 +41,10 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 
-constexpr int kTokensPerBlock = 64;
-constexpr int kTilesPerBlock = 8;  // 16-row tiles per workgroup (2 per wave)
-constexpr int kStage = 4;          // weight blocks (2 groups each) per pipeline stage
-constexpr int kStageLds = kStage * 2 * 4 * 512;  // A fragments of one stage (16 KB)
 // s_waitcnt immediate (gfx9 encoding): vmcnt 0, expcnt and lgkmcnt not waited on
 constexpr int kWaitVmcnt0 = 0x0F70;
+
+constexpr int kStage = 4;  // weight blocks (2 groups each) per pipeline stage (8 and 16 measured no faster)
 
 struct GemmParams {
     const uint8_t* tiles;
@@ -64,23 +62,22 @@ struct WStage {
     uint4 s[TPW];       // fp16 scales of the stage's 8 groups, per tile row
 };
 
-// WAVES waves per workgroup, each owning TPW = 8 / WAVES 16-row tiles (four
-// waves of two tiles measured fastest: eight waves of one tile read the
-// A operands twice as often).
-template <bool EXACT, bool SPECIAL, int WAVES>
+// Four waves per workgroup, each owning TPW 16-row tiles (at 64 tokens two
+// tiles a wave measured fastest: one reads the A operands twice as often).
+template <bool EXACT, bool SPECIAL, int TI, int TPW>
 __device__ __forceinline__ void gemm_i8_body(const GemmParams& p)
 {
-    constexpr int TPW = kTilesPerBlock / WAVES;
-    constexpr int NT = 64 * WAVES;           // threads
-    constexpr int AU = 1024 / NT;            // 16-byte activation units per thread and stage
+    constexpr int WAVES = 4;
+    constexpr int kStageLds = kStage * 2 * TI * 512;  // A fragments of one stage (4 KB a subtile)
+    constexpr int AU = kStageLds / 1024 / WAVES;      // 1 KB activation copies per wave and stage
     __shared__ __align__(16) uint8_t afrag[2][kStageLds];  // [buf][group][subtile] blocks of 512 bytes
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
     const int r = lane & 15;
     const int kq = lane >> 4;
-    const int t0 = blockIdx.y * kTokensPerBlock;
-    const int tile0 = p.tile_begin + blockIdx.x * kTilesPerBlock + wave * TPW;
+    const int t0 = blockIdx.y * (16 * TI);
+    const int tile0 = p.tile_begin + blockIdx.x * (WAVES * TPW) + wave * TPW;
     const int stages = (p.blocks + kStage - 1) / kStage;
 
     const u4* wbase[TPW];
@@ -91,9 +88,9 @@ __device__ __forceinline__ void gemm_i8_body(const GemmParams& p)
         wbase[j] = reinterpret_cast<const u4*>(p.tiles) + (size_t)tj * p.blocks * 64 + lane;
         nrow[j] = p.norms + (size_t)(tj * 16 + r) * p.groups_pad8;
     }
-    float qs[4][4];  // activation scale of token t0 + 16i + 4kq + e
+    float qs[TI][4];  // activation scale of token t0 + 16i + 4kq + e
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < TI; i++)
 #pragma unroll
         for (int e = 0; e < 4; e++) qs[i][e] = p.qscale[min(t0 + 16 * i + 4 * kq + e, p.tokens - 1)];
 
@@ -112,8 +109,8 @@ __device__ __forceinline__ void gemm_i8_body(const GemmParams& p)
         for (int j = 0; j < AU; j++) {
             const int R = AU * wave + j;
             const int b = 2 * R + (lane >> 5);
-            const int gs = b >> 2;
-            const int i = b & 3;
+            const int gs = b / TI;
+            const int i = b % TI;
             const int x = lane & 31;
             const int rr = x >> 1;
             const int pp = (x & 1) ^ ((rr >> 3) & 1) ^ (i & 1);
@@ -132,35 +129,35 @@ __device__ __forceinline__ void gemm_i8_body(const GemmParams& p)
         for (int j = 0; j < TPW; j++) ws.s[j] = *reinterpret_cast<const uint4*>(nrow[j] + st * kStage * 2);
     };
 
-    float acc[TPW][4][4];
+    float acc[TPW][TI][4];
 #pragma unroll
     for (int j = 0; j < TPW; j++)
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int i = 0; i < TI; i++)
 #pragma unroll
             for (int e = 0; e < 4; e++) acc[j][i][e] = 0.0f;
 
     // one stage: group k's A operands (four 16-token subtiles), its MFMAs
     // and its epilogue, software-pipelined so that group k+1's MFMAs and
     // group k+2's LDS reads are in flight during group k's epilogue
-    auto read_a = [&](long (&av)[4], int buf, int k) {
+    auto read_a = [&](long (&av)[TI], int buf, int k) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < TI; i++) {
             const int x = 2 * r + ((kq >> 1) ^ ((r >> 3) & 1) ^ (i & 1));
-            av[i] = *reinterpret_cast<const long*>(&afrag[buf][(k * 4 + i) * 512 + x * 16 + (kq & 1) * 8]);
+            av[i] = *reinterpret_cast<const long*>(&afrag[buf][(k * TI + i) * 512 + x * 16 + (kq & 1) * 8]);
         }
     };
-    auto issue = [&](v4i (&d)[TPW][4], const long (&av)[4], const WStage<TPW>& ws, int k) {
+    auto issue = [&](v4i (&d)[TPW][TI], const long (&av)[TI], const WStage<TPW>& ws, int k) {
         const v4i zero = {0, 0, 0, 0};
 #pragma unroll
         for (int j = 0; j < TPW; j++) {
             const u4& wc = ws.w[k >> 1][j];
             const long bop = (k & 1) ? (long)(((uint64_t)wc.w << 32) | wc.z) : (long)(((uint64_t)wc.y << 32) | wc.x);
 #pragma unroll
-            for (int i = 0; i < 4; i++) d[j][i] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[i], bop, zero, 0, 0, 0);
+            for (int i = 0; i < TI; i++) d[j][i] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[i], bop, zero, 0, 0, 0);
         }
     };
-    auto epilogue = [&](const v4i (&d)[TPW][4], const WStage<TPW>& ws, int k) {
+    auto epilogue = [&](const v4i (&d)[TPW][TI], const WStage<TPW>& ws, int k) {
 #pragma unroll
         for (int j = 0; j < TPW; j++) {
             const uint4 s4 = ws.s[j];
@@ -173,7 +170,7 @@ __device__ __forceinline__ void gemm_i8_body(const GemmParams& p)
                 hs = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(hbits)));
             asm volatile("" : "+v"(hs));  // one conversion per scale, then full-rate v_fma_f32
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+            for (int i = 0; i < TI; i++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const float df = static_cast<float>(d[j][i][e]);
@@ -186,8 +183,8 @@ __device__ __forceinline__ void gemm_i8_body(const GemmParams& p)
     };
     constexpr int KG = 2 * kStage;  // groups per stage
     auto compute = [&](const WStage<TPW>& ws, int buf, int st) {
-        long aa[2][4];
-        v4i dd[2][TPW][4];
+        long aa[2][TI];
+        v4i dd[2][TPW][TI];
         read_a(aa[0], buf, 0);
         read_a(aa[1], buf, 1);
         issue(dd[0], aa[0], ws, 0);
@@ -224,7 +221,7 @@ __device__ __forceinline__ void gemm_i8_body(const GemmParams& p)
         const int n = (tile0 + j) * 16 + r;
         if (tile0 + j >= p.tile_end || n < p.row_start || n >= p.row_end) continue;
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int i = 0; i < TI; i++)
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int t = t0 + 16 * i + 4 * kq + e;
@@ -233,23 +230,41 @@ __device__ __forceinline__ void gemm_i8_body(const GemmParams& p)
     }
 }
 
-template <bool EXACT, bool SPECIAL>
+template <bool EXACT, bool SPECIAL, int TI, int TPW>
 __global__ __launch_bounds__(256) void gemm_i8_kernel(GemmParams p)
 {
-    gemm_i8_body<EXACT, SPECIAL, 4>(p);
+    gemm_i8_body<EXACT, SPECIAL, TI, TPW>(p);
+}
+
+template <bool EXACT, int TI, int TPW>
+int32_t launch_tile(const GemmParams& p, bool special, hipStream_t stream)
+{
+    const int tiles = p.tile_end - p.tile_begin;
+    dim3 grid((tiles + 4 * TPW - 1) / (4 * TPW), (p.tokens + 16 * TI - 1) / (16 * TI));
+    if (special)
+        hipLaunchKernelGGL((gemm_i8_kernel<EXACT, true, TI, TPW>), grid, dim3(256), 0, stream, p);
+    else
+        hipLaunchKernelGGL((gemm_i8_kernel<EXACT, false, TI, TPW>), grid, dim3(256), 0, stream, p);
+    NHIP_CHECK_HIP(hipGetLastError());
+    return NHIP_OK;
 }
 
 template <bool EXACT>
 int32_t launch(const GemmParams& p, bool special, hipStream_t stream)
 {
     const int tiles = p.tile_end - p.tile_begin;
-    dim3 grid((tiles + kTilesPerBlock - 1) / kTilesPerBlock, (p.tokens + kTokensPerBlock - 1) / kTokensPerBlock);
-    if (special)
-        hipLaunchKernelGGL((gemm_i8_kernel<EXACT, true>), grid, dim3(256), 0, stream, p);
-    else
-        hipLaunchKernelGGL((gemm_i8_kernel<EXACT, false>), grid, dim3(256), 0, stream, p);
-    NHIP_CHECK_HIP(hipGetLastError());
-    return NHIP_OK;
+    const auto groups_of = [&](int ti, int tpw) {  // workgroups of a launch
+        return (int64_t)((tiles + 4 * tpw - 1) / (4 * tpw)) * ((p.tokens + 16 * ti - 1) / (16 * ti));
+    };
+    // The largest tile that leaves two workgroups for every CU.  Measured for
+    // 64 x 128 / 32 x 64 / 16 x 64, exact: 512 x 2048 x 8192 38.7 / 41.8 / - us
+    // (512 workgroups of 64 x 128); 512 x 2048 x 4096 27.2 / 22.8 / 28.3 (256);
+    // 128 x 1024 x 8192 14.4 / 8.1 / 8.6 (128; 512 of 32 x 64); 256 x 1024 x
+    // 3072 14.2 / 7.7 / 7.2 (384 of 32 x 64); 128 x 1024 x 1024 13.5 / 5.6 / 4.2;
+    // 128 x 4096 x 1024 43.7 / 15.6 / 11.5 (one chain of 128 groups a wave).
+    if (groups_of(4, 2) >= 512) return launch_tile<EXACT, 4, 2>(p, special, stream);
+    if (groups_of(2, 1) >= 512) return launch_tile<EXACT, 2, 1>(p, special, stream);
+    return launch_tile<EXACT, 1, 1>(p, special, stream);
 }
 
 }  // namespace
