@@ -548,8 +548,11 @@ int32_t nhip_ctx_info(const nhip_ctx* c, int32_t* vocab, int32_t* slots, int32_t
 int32_t nhip_step(nhip_ctx* c, const int32_t* tokens, const int32_t* row_slots, int32_t rows,
                   const int32_t* head_rows, int32_t heads, float* logits, int32_t k, int32_t* topk_idx,
                   float* topk_lp, int32_t* argmax);
-/* FeedSlot (Engine.cs:2285-2301): `count` tokens into one slot in steps of
- * `chunk` rows; logits [vocab] of the last token if non-NULL. */
+/* FeedSlot (Engine.cs:2285-2301): `count` tokens into one slot, logits [vocab]
+ * of the last token if non-NULL.  Prompts longer than `chunk` go in equal steps
+ * of up to 512 rows (fewer for a smaller context or very many attention
+ * chunks), with the results of any other cut; if a token is out of range,
+ * those before its chunk of `chunk` tokens are fed. */
 int32_t nhip_slot_feed(nhip_ctx* c, int32_t slot, const int32_t* tokens, int32_t count, float* logits);
 /* ResetSlot / MarkSlot / RewindSlot / SlotLength (BatchEngine.cs:24-29,
  * Engine.cs:2224-2283): reset clears the slot's histories and sets its length

@@ -60,6 +60,11 @@ constexpr int kPer = kMaxDim / kThreads;    // elements of a dim-row per thread:
 constexpr int kMaxStream = kLanes * kMaxDim;
 constexpr int kCondPer = 8 * kMaxDim / kThreads;  // condition-weight entries per thread
 constexpr int kHistPer = (2560 + kThreads - 1) / kThreads;  // Q/K/V frame entries per thread (qw + kw + vw <= 2560)
+// A FeedSlot step's rows (the results do not depend on how a prompt is cut):
+// the row kernels run one workgroup per row, so a 64-row step leaves 3/4 of the
+// CUs idle in most of a layer's launches.  Needle 3, a 300-token prompt: 5.62 ms
+// in five steps of up to 64 rows, 1.94 ms in one.
+constexpr int kMaxFeedRows = 512;
 constexpr int kMaxPhiGroups = kLanes * kMaxDim / 128;       // groups of a phi row (K = 4 * dim)
 
 __device__ __forceinline__ float sigmoid_poly(float x) { return 1.0f / (1.0f + exp_poly(-x)); }
@@ -1386,6 +1391,8 @@ struct nhip_ctx {
     int site_count = 0, sites[16] = {};
     uint64_t global_mask = 0;
     int slots = 0, capacity = 0, max_rows = 0, max_chunks = 0;
+    int feed_rows = 0;  // rows of a FeedSlot step (>= max_rows); the scratch holds that many
+    int in_stride = 0;  // of the current step's inputs: max_rows, or feed_rows for a longer step
     // weights
     nhip_weights* embedding = nullptr;
     const uint8_t* embedding_raw = nullptr;
@@ -1405,14 +1412,14 @@ struct nhip_ctx {
     float *qkv_hist = nullptr, *engram_hist = nullptr, *snap_qkv = nullptr, *snap_engram = nullptr;
     std::vector<int32_t> len, marked, prev, snap_prev;
     float *rope_cos = nullptr, *rope_sin = nullptr;
-    // scratch for max_rows rows (stream_a holds the embedding, the layers
+    // scratch for feed_rows rows, logits for max_rows (stream_a holds the embedding, the layers
     // alternate between the two stream buffers)
     float *stream_a = nullptr, *stream_b = nullptr, *normed = nullptr, *input = nullptr, *residual = nullptr,
           *raw = nullptr, *gate = nullptr, *att = nullptr, *proj = nullptr, *key = nullptr, *stage = nullptr,
           *ein = nullptr, *post_gate = nullptr, *mix = nullptr, *qs = nullptr, *logits = nullptr, *act_s = nullptr,
           *act_o = nullptr, *act4_s = nullptr, *act4_o = nullptr;
     int8_t *act_v = nullptr, *act4_v = nullptr, *q8 = nullptr;  // act4: the stream's 4-bit Prepare (phi input)
-    int32_t* d_in = nullptr;  // the per-row inputs of a step, kInSections x max_rows, then the engram rows
+    int32_t* d_in = nullptr;  // the per-row inputs of a step, kInSections x in_stride, then the engram rows
     int32_t* h_in = nullptr;  // their pinned host staging
     void* attn_ws = nullptr;
     size_t attn_ws_bytes = 0;
@@ -1444,8 +1451,8 @@ enum {
     kInSections
 };
 
-int32_t* in(nhip_ctx* c, int32_t* base, int section) { return base + (size_t)section * c->max_rows; }
-int32_t* in_erows(nhip_ctx* c, int32_t* base) { return base + (size_t)kInSections * c->max_rows; }
+int32_t* in(nhip_ctx* c, int32_t* base, int section) { return base + (size_t)section * c->in_stride; }
+int32_t* in_erows(nhip_ctx* c, int32_t* base) { return base + (size_t)kInSections * c->in_stride; }
 
 template <typename T>
 int32_t ctx_alloc(nhip_ctx* c, T** p, size_t count)
@@ -1749,7 +1756,14 @@ int32_t load_model(nhip_ctx* c)
 
 int32_t alloc_state(nhip_ctx* c)
 {
-    const int d = c->dim, R = c->max_rows, qw = c->heads * c->qk, kw = c->kv * c->qk, vw = c->kv * c->vd,
+    // FeedSlot's steps: as many rows as fill the chip's CUs with the row
+    // kernels' one workgroup per row, within the context and 64 MB of attention
+    // partials
+    c->feed_rows = std::max(c->max_rows, std::min(c->capacity, kMaxFeedRows));
+    while (c->feed_rows > c->max_rows &&
+           nhip_attention_decode_workspace(c->feed_rows, c->heads, c->max_chunks) > (size_t)64 << 20)
+        c->feed_rows = std::max(c->max_rows, c->feed_rows / 2);
+    const int d = c->dim, R = c->feed_rows, HR = c->max_rows, qw = c->heads * c->qk, kw = c->kv * c->qk, vw = c->kv * c->vd,
               ow = c->heads * c->vd, all = qw + kw + vw, sw = kLanes * d;
     const size_t cells = (size_t)c->layers * c->slots * c->capacity;
     const size_t hist = (size_t)c->layers * c->slots * 2 * all;
@@ -1772,9 +1786,9 @@ int32_t alloc_state(nhip_ctx* c)
         (rc = ctx_alloc(c, &c->act4_s, (size_t)R * stride4)) || (rc = ctx_alloc(c, &c->act4_o, (size_t)R * stride4)) ||
         (rc = ctx_alloc(c, &c->post_gate, (size_t)R * 4)) || (rc = ctx_alloc(c, &c->mix, (size_t)R * 16)) ||
         (rc = ctx_alloc(c, &c->q8, (size_t)R * qw)) || (rc = ctx_alloc(c, &c->qs, (size_t)R * c->heads)) ||
-        (rc = ctx_alloc(c, &c->logits, (size_t)R * c->vocab)) || (rc = ctx_alloc(c, &c->act_v, (size_t)R * sw)) ||
-        (rc = ctx_alloc(c, &c->d_topk_idx, (size_t)R * 8)) || (rc = ctx_alloc(c, &c->d_topk_lp, (size_t)R * 8)) ||
-        (rc = ctx_alloc(c, &c->d_argmax, (size_t)R)) ||
+        (rc = ctx_alloc(c, &c->logits, (size_t)HR * c->vocab)) || (rc = ctx_alloc(c, &c->act_v, (size_t)R * sw)) ||
+        (rc = ctx_alloc(c, &c->d_topk_idx, (size_t)HR * 8)) || (rc = ctx_alloc(c, &c->d_topk_lp, (size_t)HR * 8)) ||
+        (rc = ctx_alloc(c, &c->d_argmax, (size_t)HR)) ||
         (rc = ctx_alloc(c, &c->act_s, (size_t)R * stride4)) || (rc = ctx_alloc(c, &c->act_o, (size_t)R * stride4)) ||
         (rc = ctx_alloc(c, &c->d_in, (size_t)R * (kInSections + std::max(c->engram_tables, 1)))))
         return rc;
@@ -1784,7 +1798,7 @@ int32_t alloc_state(nhip_ctx* c)
     c->attn_ws_bytes = nhip_attention_decode_workspace(R, c->heads, c->max_chunks);
     NHIP_CHECK_HIP(hipMalloc(&c->attn_ws, c->attn_ws_bytes));
     c->allocations.push_back(c->attn_ws);
-    c->topk_ws_bytes = nhip_topk_lse_workspace(R, c->vocab);
+    c->topk_ws_bytes = nhip_topk_lse_workspace(HR, c->vocab);
     NHIP_CHECK_HIP(hipMalloc(&c->topk_ws, c->topk_ws_bytes));
     c->allocations.push_back(c->topk_ws);
     // EngineCore.RopeFrequencies + BuildRopeTables (Engine.cs:336-356):
@@ -2186,85 +2200,16 @@ int32_t snapshot_slot(nhip_ctx* c, int slot, bool to_snapshot)
     return NHIP_OK;
 }
 
-}  // namespace
-
-extern "C" {
-
-int32_t nhip_ctx_destroy(nhip_ctx* c)
-{
-    clear_error();
-    if (!c) return NHIP_OK;
-    if (c->stream_h) (void)hipStreamSynchronize(c->stream_h);
-    for (nhip_ctx::Graph& g : c->graphs) (void)hipGraphExecDestroy(g.exec);
-    for (void* p : c->allocations) (void)hipFree(p);
-    for (nhip_weights* w : c->stacked) (void)nhip_weights_destroy(w);
-    if (c->h_in) (void)hipHostFree(c->h_in);
-    if (c->stream_h) (void)hipStreamDestroy(c->stream_h);
-    delete c;
-    return NHIP_OK;
-}
-
-int32_t nhip_ctx_create(const nhip_model* model, int32_t capacity, int32_t slots, int32_t chunk, int32_t max_chunks,
-                        nhip_ctx** out)
-{
-    clear_error();
-    NHIP_REQUIRE(model && out, "null argument");
-    *out = nullptr;
-    if (chunk <= 0) chunk = 64;
-    if (max_chunks <= 0) max_chunks = 8;
-    // BatchedEngine's limits (BatchEngine.cs:11-12): 1..16 slots
-    NHIP_REQUIRE(capacity > 0 && slots >= 1 && slots <= 16 && chunk <= 4096 && max_chunks <= 256,
-                 "capacity %d, slots %d (1..16), chunk %d (<= 4096), max_chunks %d (<= 256)", capacity, slots, chunk,
-                 max_chunks);
-    int32_t rc = ensure_device();
-    if (rc) return rc;
-    nhip_ctx* c = new nhip_ctx();
-    c->model = model;
-    c->slots = slots;
-    c->capacity = capacity;
-    c->max_rows = chunk;
-    c->max_chunks = max_chunks;
-    if (hipStreamCreateWithFlags(&c->stream_h, hipStreamNonBlocking) != hipSuccess) {
-        delete c;
-        set_error("hipStreamCreateWithFlags failed");
-        return NHIP_ERR_HIP;
-    }
-    if ((rc = load_model(c)) || (rc = alloc_state(c))) {
-        const std::string why = nhip_last_error();
-        nhip_ctx_destroy(c);
-        set_error("%s", why.c_str());
-        return rc;
-    }
-    if (hipStreamSynchronize(c->stream_h) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
-        nhip_ctx_destroy(c);
-        set_error("context set-up failed");
-        return NHIP_ERR_HIP;
-    }
-    *out = c;
-    return NHIP_OK;
-}
-
-int32_t nhip_ctx_info(const nhip_ctx* c, int32_t* vocab, int32_t* slots, int32_t* capacity, int32_t* chunk)
-{
-    clear_error();
-    NHIP_REQUIRE(c, "null context");
-    if (vocab) *vocab = c->vocab;
-    if (slots) *slots = c->slots;
-    if (capacity) *capacity = c->capacity;
-    if (chunk) *chunk = c->max_rows;
-    return NHIP_OK;
-}
-
-int32_t nhip_step(nhip_ctx* c, const int32_t* tokens, const int32_t* row_slots, int32_t rows, const int32_t* head_rows,
+// ForwardBatch (Engine.cs:2303-2350) over 1 to feed_rows rows, at most max_rows
+// of them head rows.
+int32_t step_rows(nhip_ctx* c, const int32_t* tokens, const int32_t* row_slots, int32_t rows, const int32_t* head_rows,
                   int32_t heads, float* logits, int32_t k, int32_t* topk_idx, float* topk_lp, int32_t* argmax)
 {
-    clear_error();
-    NHIP_REQUIRE(c && tokens && row_slots, "null argument");
-    // ForwardBatch's checks (Engine.cs:2305-2307)
-    NHIP_REQUIRE(rows >= 1 && rows <= c->max_rows, "rows %d outside [1, %d]", rows, c->max_rows);
     NHIP_REQUIRE(heads >= 0 && heads <= rows && (heads == 0 || head_rows), "heads %d outside [0, %d]", heads, rows);
     NHIP_REQUIRE(k >= 0 && k <= 8 && (k == 0 || (topk_idx && topk_lp)), "k %d outside [0, 8] or null top-k output", k);
-    const int R = c->max_rows;
+    // (the stride follows from the row count, which is part of a graph's key)
+    c->in_stride = rows <= c->max_rows ? c->max_rows : c->feed_rows;
+    const int R = c->in_stride;
     int32_t* h = c->h_in;
     std::vector<char> seen(c->slots, 0);
     bool single_runs = true;  // every row the only row of its slot
@@ -2380,6 +2325,85 @@ int32_t nhip_step(nhip_ctx* c, const int32_t* tokens, const int32_t* row_slots, 
     return NHIP_OK;
 }
 
+}  // namespace
+
+extern "C" {
+
+int32_t nhip_ctx_destroy(nhip_ctx* c)
+{
+    clear_error();
+    if (!c) return NHIP_OK;
+    if (c->stream_h) (void)hipStreamSynchronize(c->stream_h);
+    for (nhip_ctx::Graph& g : c->graphs) (void)hipGraphExecDestroy(g.exec);
+    for (void* p : c->allocations) (void)hipFree(p);
+    for (nhip_weights* w : c->stacked) (void)nhip_weights_destroy(w);
+    if (c->h_in) (void)hipHostFree(c->h_in);
+    if (c->stream_h) (void)hipStreamDestroy(c->stream_h);
+    delete c;
+    return NHIP_OK;
+}
+
+int32_t nhip_ctx_create(const nhip_model* model, int32_t capacity, int32_t slots, int32_t chunk, int32_t max_chunks,
+                        nhip_ctx** out)
+{
+    clear_error();
+    NHIP_REQUIRE(model && out, "null argument");
+    *out = nullptr;
+    if (chunk <= 0) chunk = 64;
+    if (max_chunks <= 0) max_chunks = 8;
+    // BatchedEngine's limits (BatchEngine.cs:11-12): 1..16 slots
+    NHIP_REQUIRE(capacity > 0 && slots >= 1 && slots <= 16 && chunk <= 4096 && max_chunks <= 256,
+                 "capacity %d, slots %d (1..16), chunk %d (<= 4096), max_chunks %d (<= 256)", capacity, slots, chunk,
+                 max_chunks);
+    int32_t rc = ensure_device();
+    if (rc) return rc;
+    nhip_ctx* c = new nhip_ctx();
+    c->model = model;
+    c->slots = slots;
+    c->capacity = capacity;
+    c->max_rows = chunk;
+    c->max_chunks = max_chunks;
+    if (hipStreamCreateWithFlags(&c->stream_h, hipStreamNonBlocking) != hipSuccess) {
+        delete c;
+        set_error("hipStreamCreateWithFlags failed");
+        return NHIP_ERR_HIP;
+    }
+    if ((rc = load_model(c)) || (rc = alloc_state(c))) {
+        const std::string why = nhip_last_error();
+        nhip_ctx_destroy(c);
+        set_error("%s", why.c_str());
+        return rc;
+    }
+    if (hipStreamSynchronize(c->stream_h) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
+        nhip_ctx_destroy(c);
+        set_error("context set-up failed");
+        return NHIP_ERR_HIP;
+    }
+    *out = c;
+    return NHIP_OK;
+}
+
+int32_t nhip_ctx_info(const nhip_ctx* c, int32_t* vocab, int32_t* slots, int32_t* capacity, int32_t* chunk)
+{
+    clear_error();
+    NHIP_REQUIRE(c, "null context");
+    if (vocab) *vocab = c->vocab;
+    if (slots) *slots = c->slots;
+    if (capacity) *capacity = c->capacity;
+    if (chunk) *chunk = c->max_rows;
+    return NHIP_OK;
+}
+
+int32_t nhip_step(nhip_ctx* c, const int32_t* tokens, const int32_t* row_slots, int32_t rows, const int32_t* head_rows,
+                  int32_t heads, float* logits, int32_t k, int32_t* topk_idx, float* topk_lp, int32_t* argmax)
+{
+    clear_error();
+    NHIP_REQUIRE(c && tokens && row_slots, "null argument");
+    // ForwardBatch's checks (Engine.cs:2305-2307)
+    NHIP_REQUIRE(rows >= 1 && rows <= c->max_rows, "rows %d outside [1, %d]", rows, c->max_rows);
+    return step_rows(c, tokens, row_slots, rows, head_rows, heads, logits, k, topk_idx, topk_lp, argmax);
+}
+
 int32_t nhip_slot_feed(nhip_ctx* c, int32_t slot, const int32_t* tokens, int32_t count, float* logits)
 {
     clear_error();
@@ -2388,13 +2412,22 @@ int32_t nhip_slot_feed(nhip_ctx* c, int32_t slot, const int32_t* tokens, int32_t
     NHIP_REQUIRE(count >= 0, "count %d", count);
     // FeedSlot (Engine.cs:2285-2301): the capacity is checked before any work
     NHIP_REQUIRE(c->len[slot] + count <= c->capacity, "slot %d: context capacity %d exceeded", slot, c->capacity);
-    std::vector<int32_t> row_slots(c->max_rows, slot);
-    for (int start = 0; start < count; start += c->max_rows) {
-        const int n = std::min(c->max_rows, count - start);
+    // equal steps of at most feed_rows rows; a prompt with a bad token goes in
+    // steps of the context's chunk, which feed what comes before that chunk
+    bool valid = true;
+    for (int i = 0; i < count; i++) valid = valid && tokens[i] >= 0 && tokens[i] < c->vocab;
+    int rows = c->max_rows;
+    if (valid && count > c->max_rows) {
+        const int steps = (count + c->feed_rows - 1) / c->feed_rows;
+        rows = (count + steps - 1) / steps;
+    }
+    std::vector<int32_t> row_slots(rows, slot);
+    for (int start = 0; start < count; start += rows) {
+        const int n = std::min(rows, count - start);
         const bool last = start + n == count;
         const int32_t head = n - 1;
         const int heads = last && logits ? 1 : 0;
-        const int32_t rc = nhip_step(c, tokens + start, row_slots.data(), n, heads ? &head : nullptr, heads,
+        const int32_t rc = step_rows(c, tokens + start, row_slots.data(), n, heads ? &head : nullptr, heads,
                                      heads ? logits : nullptr, 0, nullptr, nullptr, nullptr);
         if (rc) return rc;
     }
