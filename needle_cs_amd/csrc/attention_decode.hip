@@ -592,6 +592,311 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(ATTN_HEAD_PARAMS, Deco
     *dst = sum * (1.0f / total);
 }
 
+// Attention of many rows (prompts): one workgroup of T threads per (row, kv
+// head) runs every chunk of the row's plan for the group's query heads and the
+// merge, with the chunk kernel's and decode_merge_kernel's arithmetic per
+// output, so the results are the same bits.
+//   scores   one v_mfma_i32_16x16x64_i8 per 16 positions: A the group's heads
+//            (a lane's 16 query bytes straight from memory, zeros past the
+//            group and past qk 48), B the positions' key bytes; lane (r, kq)
+//            then holds position r's dots of heads 4kq..+3
+//   peaks    of position quads beside the scores, then a thread per (chunk, head)
+//   weights  e_s and e_s * valueScale_s, all positions in parallel; the chunk
+//            weights of the merge by a wave per head
+//   sums     a thread per (chunk, head) adds its e_s in ascending order
+//   values   a thread per (chunk, HPT heads, 4 dims) walks the chunk's
+//            positions: a value dword is converted once for HPT heads; chunks
+//            go in rounds of as many as the workgroup has threads for, each
+//            round merged by a thread per (head, dim) before the next
+// What bounds it: the value walk's VALU work, a multiply and an add per
+// (position, head, dim) and 1 / HPT of the conversions (half of the time of
+// 128 rows of 1024 positions), and the latencies of the phases before it.
+// Measured, with the launch it replaces (and its merge): 128 rows of up to 1024
+// positions, 12 heads on 2, up to 64 chunks 19.7 us (45.3); 300 rows of up to
+// 300, 8 chunks 14.5 (25.8); 2 x 128 rows, 8 heads on 8, 64 chunks 43.0 (57.6).
+constexpr int kGroupMaxLds = 160 * 1024;
+constexpr int group_chunks_per_round(int T, int group, int hpt) { return T / (16 * ((group + hpt - 1) / hpt)); }
+constexpr int group_row_ld(int capacity) { return ((capacity + 15) & ~15) + 4; }
+// LDS bytes: scores / e_s and e_s * valueScale_s of every head and position,
+// two rounds' partials, three words per (chunk, head) and one per head
+size_t group_lds(int capacity, int max_chunks, int T, int group, int hpt)
+{
+    const int chunks = std::min(max_chunks, std::max(capacity / 16, 1));
+    return sizeof(float) * ((size_t)2 * group * group_row_ld(capacity) +
+                            (size_t)2 * group_chunks_per_round(T, group, hpt) * group * 64 +
+                            (size_t)3 * chunks * group + group);
+}
+
+template <int T, int HPT>
+__global__ __launch_bounds__(T) void group_attention_kernel(ATTN_HEAD_PARAMS, DecodeAttnParams p)
+{
+    ATTN_TAKE_HEAD(p, q, qscale);
+    typedef int v4i __attribute__((ext_vector_type(4)));
+    constexpr int W = T / 64;
+    constexpr int MI = (kMaxHeadsPerBlock * 64 + T - 1) / T;  // (head, dim) outputs a thread merges
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int row = blockIdx.x;
+    const int kvh = blockIdx.y;
+    const int group = p.heads / p.kv_heads;
+    const int h0 = kvh * group;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int slot = uniform_load(p.row_slot, row);
+    const int first = uniform_load(p.row_first, row);
+    const int count = uniform_load(p.row_count, row);
+    asm volatile("" ::"s"(p.keys), "s"(p.kscale), "s"(p.values), "s"(p.vscale), "s"(p.qk), "s"(p.inv_sqrt),
+                 "s"(p.slots), "s"(p.capacity), "s"(p.max_chunks), "s"(p.out));
+    float* out = p.out + ((size_t)row * p.heads + h0) * 64;
+    // rows with an invalid slot or span produce zeros (no out-of-range reads)
+    if (!((slot >= 0) & (slot < p.slots) & (first >= 0) & (count >= 1) & (count <= p.capacity - first) &
+          (count <= p.lmax))) {
+        for (int i = tid; i < group * 64; i += T) out[i] = 0.0f;
+        return;
+    }
+    int length;
+    const int needed = plan(count, p.max_chunks, &length);
+    const uint32_t mag_len = length <= 256 ? magic((uint32_t)length) : 0u;
+    auto chunk_of = [&](int s) { return mag_len ? fast_div(s, mag_len) : s / length; };
+    const int ld = group_row_ld(p.lmax);
+    const int S = (group + HPT - 1) / HPT;
+    const int C = T / (16 * S);
+    float* sc = reinterpret_cast<float*>(lds);        // [group][ld] scores, then e_s
+    float* wl = sc + group * ld;                      // [group][ld] e_s * valueScale_s
+    uint32_t* quad = reinterpret_cast<uint32_t*>(wl); // [group][ld / 4] peaks of position quads, until wl is written
+    float* part = wl + group * ld;                    // [2][C][group][64]
+    float* pk = part + 2 * C * group * 64;            // [needed][group] chunk peaks
+    float* cs = pk + needed * group;                  // [needed][group] chunk sums
+    float* wt = cs + needed * group;                  // [needed][group] chunk weights
+    float* tot = wt + needed * group;                 // [group]
+
+    // scores
+    const int qk = p.qk;
+    const int r = lane & 15;
+    const int kq = lane >> 4;
+    const size_t cell0 = ((size_t)slot * p.capacity + first) * p.kv_heads + kvh;
+    const int8_t* kbase = p.keys + cell0 * qk;
+    const float* ksb = p.kscale + cell0;
+    const float* vsb = p.vscale + cell0;
+    const bool live = r < group && 16 * kq < qk;
+    v4i a = *reinterpret_cast<const v4i*>(p.q + ((size_t)row * p.heads + h0 + min(r, group - 1)) * qk +
+                                          min(16 * kq, qk - 16));
+    if (!live) a = v4i{0, 0, 0, 0};
+    float qs[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) qs[i] = p.qscale[(size_t)row * p.heads + h0 + min(4 * kq + i, group - 1)] * p.inv_sqrt;
+    const float vs0 = vsb[(size_t)min(tid, count - 1) * p.kv_heads];
+    const int tiles = (count + 15) >> 4;
+    constexpr int KT = 4;  // tiles a wave loads together
+    for (int t = wave; t < tiles; t += KT * W) {
+        v4i b[KT];
+        float ks[KT];
+#pragma unroll
+        for (int j = 0; j < KT; j++) {
+            const size_t c = (size_t)min(16 * (t + j * W) + r, count - 1) * p.kv_heads;
+            b[j] = *reinterpret_cast<const v4i*>(kbase + c * qk + min(16 * kq, qk - 16));
+            ks[j] = ksb[c];
+        }
+#pragma unroll
+        for (int j = 0; j < KT; j++) {
+            const v4i zero = {0, 0, 0, 0};
+            const v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b[j], zero, 0, 0, 0);
+            const int s = 16 * (t + j * W) + r;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float x = (static_cast<float>(d[i]) * ks[j]) * qs[i];
+                // the peak of the aligned quad of positions: chunks begin at
+                // multiples of 4
+                uint32_t key = order_key(s < count ? x : -INFINITY);
+                key = max(key, lane_xor<1>(key));
+                key = max(key, lane_xor<2>(key));
+                if (s < count && 4 * kq + i < group) {
+                    sc[(4 * kq + i) * ld + s] = x;
+                    if ((r & 3) == 0) quad[(4 * kq + i) * (ld / 4) + (s >> 2)] = key;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    // chunk peaks (maxima are order-free)
+    for (int u = tid; u < needed * group; u += T) {
+        const int c = u / group, h = u - c * group;
+        const int q0 = c * length >> 2, q1 = min(c * length + length + 3, count + 3) >> 2;
+        uint32_t key = order_key(-INFINITY);
+        for (int x = q0; x < q1; x++) key = max(key, quad[h * (ld / 4) + x]);
+        pk[u] = order_value(key);
+    }
+    __syncthreads();
+    // e_s, e_s * valueScale_s
+    for (int s = tid; s < count; s += T) {
+        const float vs = s == tid ? vs0 : vsb[(size_t)s * p.kv_heads];
+        const int c = chunk_of(s);
+        for (int h = 0; h < group; h++) {
+            const float e = exp_poly(sc[h * ld + s] - pk[c * group + h]);
+            sc[h * ld + s] = e;
+            wl[h * ld + s] = e * vs;
+        }
+    }
+    // the merge's chunk weights, a wave per head (as decode_merge_kernel)
+    for (int h = wave; h < group; h += W) {
+        float v[4], peak = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int c = lane + 64 * j;
+            v[j] = pk[min(c, needed - 1) * group + h];
+            if (c < needed) peak = ref_max(peak, v[j]);
+        }
+        peak = wave_max(peak);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int c = lane + 64 * j;
+            if (c < needed) wt[c * group + h] = exp_poly(v[j] - peak);
+        }
+    }
+    __syncthreads();
+    // chunk sums
+    for (int u = tid; u < needed * group; u += T) {
+        const int c = u / group, h = u - c * group;
+        const int begin = c * length, n = min(length, count - begin);
+        const float* e = sc + h * ld + begin;
+        float total = 0.0f;
+        int s = 0;
+        for (; s + 4 <= n; s += 4) {
+            const float4 v = *reinterpret_cast<const float4*>(e + s);
+            total = total + v.x;
+            total = total + v.y;
+            total = total + v.z;
+            total = total + v.w;
+        }
+        for (; s < n; s++) total = total + e[s];
+        cs[u] = total;
+    }
+    // values, C chunks a round; a round's first value dwords load before the
+    // round ahead of it is merged
+    const int cl = tid / (16 * S);
+    const int sg = (tid - cl * 16 * S) >> 4;
+    const int dq = tid & 15;
+    const uint8_t* vbase = reinterpret_cast<const uint8_t*>(p.values) + cell0 * 64 + 4 * dq;
+    const uint32_t vrow = (uint32_t)p.kv_heads * 64u;
+    float msum[MI];
+#pragma unroll
+    for (int m = 0; m < MI; m++) msum[m] = 0.0f;
+    constexpr int VB = 20;  // value dwords loaded together (a 16-position plan's usual chunk)
+    uint32_t v[VB];
+    auto span_of = [&](int c0, int& begin, int& L) {
+        const int c = c0 + cl;
+        const bool on = cl < C && c < needed;
+        begin = on ? c * length : 0;
+        L = on ? min(length, count - begin) : 0;
+        return on;
+    };
+    auto vload = [&](int begin, int L, int s0) {
+        const uint8_t* vb = vbase + (size_t)begin * vrow;
+#pragma unroll
+        for (int j = 0; j < VB; j++)
+            v[j] = *reinterpret_cast<const uint32_t*>(vb + (size_t)(uint32_t)min(s0 + j, max(L - 1, 0)) * vrow);
+    };
+    int begin, L;
+    bool on = span_of(0, begin, L);
+    vload(begin, L, 0);
+    for (int c0 = 0, buf = 0; c0 < needed; c0 += C, buf ^= 1) {
+        float o[HPT][4];
+        const float* w[HPT];
+#pragma unroll
+        for (int k = 0; k < HPT; k++) {
+            w[k] = wl + min(sg * HPT + k, group - 1) * ld + begin;
+#pragma unroll
+            for (int d = 0; d < 4; d++) o[k][d] = 0.0f;
+        }
+        const int lq = max((L - 1) & ~3, 0);  // the chunk's last quad
+        for (int s0 = 0; __any(s0 < L); s0 += VB) {
+            if (s0 > 0) vload(begin, L, s0);
+#pragma unroll
+            for (int j4 = 0; j4 < VB; j4 += 4) {
+                if (!__any(s0 + j4 < L)) break;
+                float4 w4[HPT];
+#pragma unroll
+                for (int k = 0; k < HPT; k++) w4[k] = *reinterpret_cast<const float4*>(w[k] + min(s0 + j4, lq));
+                // a chunk's positions end inside a quad, or a lane's chunk
+                // before the others': weights of 0 add +-0 to sums that are
+                // never -0
+                const int rem = L - (s0 + j4);
+                if (!__all(rem >= 4)) {
+#pragma unroll
+                    for (int k = 0; k < HPT; k++) {
+                        w4[k].x = rem > 0 ? w4[k].x : 0.0f;
+                        w4[k].y = rem > 1 ? w4[k].y : 0.0f;
+                        w4[k].z = rem > 2 ? w4[k].z : 0.0f;
+                        w4[k].w = rem > 3 ? w4[k].w : 0.0f;
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const uint32_t x = v[j4 + j];
+                    const float f[4] = {sx8(x, 0), sx8(x, 1), sx8(x, 2), sx8(x, 3)};
+#pragma unroll
+                    for (int k = 0; k < HPT; k++) {
+                        const float ww = j == 0 ? w4[k].x : j == 1 ? w4[k].y : j == 2 ? w4[k].z : w4[k].w;
+#pragma unroll
+                        for (int d = 0; d < 4; d++) o[k][d] = o[k][d] + ww * f[d];
+                    }
+                }
+            }
+        }
+        float* pb = part + buf * C * group * 64;
+        if (on) {
+#pragma unroll
+            for (int k = 0; k < HPT; k++)
+                if (sg * HPT + k < group)
+                    *reinterpret_cast<float4*>(pb + (cl * group + sg * HPT + k) * 64 + 4 * dq) =
+                        make_float4(o[k][0], o[k][1], o[k][2], o[k][3]);
+        }
+        on = span_of(c0 + C, begin, L);
+        vload(begin, L, 0);
+        // one barrier a round: the merge below reads this buffer, and the next
+        // write to it is two rounds ahead.  (The first also publishes the
+        // chunk sums.)
+        __syncthreads();
+        const int n = min(C, needed - c0);
+#pragma unroll
+        for (int m = 0; m < MI; m++) {
+            const int i = tid + m * T;
+            if (i < group * 64) {
+                const float* wh = wt + c0 * group + (i >> 6);
+                constexpr int MB = 8;
+                for (int j0 = 0; j0 < n; j0 += MB) {
+                    float ww[MB], av[MB];
+#pragma unroll
+                    for (int j = 0; j < MB; j++) {
+                        const int jj = min(j0 + j, n - 1);
+                        ww[j] = wh[jj * group];
+                        av[j] = pb[jj * group * 64 + i];
+                    }
+#pragma unroll
+                    for (int j = 0; j < MB; j++) {
+                        if (j0 + j >= n) break;  // uniform
+                        // (MergePartials' two-chunk branch starts from the first product)
+                        msum[m] = needed == 2 && c0 + j0 + j == 0 ? ww[j] * av[j] : msum[m] + ww[j] * av[j];
+                    }
+                }
+            }
+        }
+        if (c0 == 0) {  // the heads' totals, a wave each from the last one down
+            for (int h = W - 1 - wave; h < group; h += W) {
+                float total = 0.0f;
+                for (int c = 0; c < needed; c++) total = total + wt[c * group + h] * cs[c * group + h];
+                if (lane == 0) tot[h] = total;
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < MI; m++) {
+        const int i = tid + m * T;
+        if (i < group * 64) out[i] = msum[m] * (1.0f / tot[i >> 6]);
+    }
+}
+
 // Whole-row attention for caches of at most kRowMaxCapacity positions: one
 // workgroup per (row, query head) runs every chunk of the row's plan and then
 // merges them itself, with the chunk kernel's per-chunk arithmetic and
@@ -1443,13 +1748,80 @@ int32_t attention_decode_needle3_impl(const Needle3AttnInputs& in, int32_t rows,
     return NHIP_OK;
 }
 
+template <int T, int HPT>
+int32_t launch_group(const DecodeAttnParams& p, size_t lds, hipStream_t stream)
+{
+    static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(&group_attention_kernel<T, HPT>),
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kGroupMaxLds);
+    NHIP_CHECK_HIP(set);
+    hipLaunchKernelGGL((group_attention_kernel<T, HPT>), dim3(p.rows, p.kv_heads), dim3(T), lds, stream,
+                       ATTN_HEAD_ARGS(p, p.q, p.qscale), p);
+    NHIP_CHECK_HIP(hipGetLastError());
+    return NHIP_OK;
+}
+
+template <int T>
+int32_t launch_group_hpt(const DecodeAttnParams& p, int hpt, size_t lds, hipStream_t stream)
+{
+    return hpt == 3 ? launch_group<T, 3>(p, lds, stream)
+                    : hpt == 2 ? launch_group<T, 2>(p, lds, stream) : launch_group<T, 1>(p, lds, stream);
+}
+
+// The group kernel for batches of many rows whose spans are at most max_count
+// positions (0: unknown, up to the capacity); 1 when it does not take them.
+// The others are faster (here, there):
+//  - while their workgroups, one per (row, chunk), are few: 20 rows of up to
+//    1024 positions in up to 63 chunks, 12 heads on 2, 18.2 and 12.5 us, but 64
+//    rows 18.6 and 27.4; 64 rows in up to 8 chunks 10.3 and 9.6;
+//  - over short caches (the whole-row kernel) for one head per kv head or few
+//    (row, head) pairs: 66 rows, 8 heads on 4, 300 positions 8.6 and 6.1, but
+//    180 rows, 12 on 2, 170 positions 10.4 and 13.0;
+//  - when the rows read caches of their own, which only the chunk kernel reads
+//    in whole cache rows: 96 rows, 16 heads on 8, 2048 positions 55.7 and 38.6;
+//    16 on 16 78 and 46, but 100 rows, 12 on 2, 1024 positions 17.8 and 26.5;
+//  - past 1024 positions with one head per kv head (100 rows, 8 heads, 2000
+//    positions 51 and 43; 2 x 128 rows, 1024 positions 43.6 and 57.5), and where
+//    LDS leaves one workgroup a CU: 128 rows, 16 on 8, 4096 positions 145 and
+//    101, but 140 rows, 8 on 4 22.9 and 28.9.
+// T: 1024 threads while every workgroup has a CU of its own (128 rows of up to
+// 1024, 12 on 2, 64 chunks: 19.7 us, 512 threads 24.3), then 512, or 256 for
+// short spans and few chunks (300 rows of up to 300, 8 chunks: 14.5 us, 512
+// threads 15.8).  HPT: the most heads a thread that keep the threads busy (300
+// rows of up to 1024 in 8 chunks, 512 threads: 2 heads 40 us with 3/4 of them,
+// 3 heads 54 with half, 1 head 52).
+int32_t launch_group_attention(DecodeAttnParams p, int32_t max_count, hipStream_t stream)
+{
+    const int group = p.heads / p.kv_heads;
+    const int span = max_count > 0 ? std::min(max_count, p.capacity) : p.capacity;
+    const int chunks = std::min(p.max_chunks, std::max(span / 16, 1));
+    if (p.rows <= kPlacedRows && p.rows * chunks <= 2560) return 1;
+    if (p.capacity <= kRowMaxCapacity && (group == 1 || (int64_t)p.rows * p.heads < 1024)) return 1;
+    const int64_t blocks = (int64_t)p.rows * p.kv_heads;
+    const bool own = p.rows < 8 * (int64_t)p.slots;  // few rows a slot
+    if (own && (group == 1 || span > 1024 || blocks > 1024)) return 1;
+    if (group == 1 && span > 1024) return 1;
+    const int T = blocks <= p.cus ? 1024 : span > 384 && chunks * 16 * group >= 512 ? 512 : 256;
+    const auto fills = [&](int hpt, float share) {
+        return group % hpt == 0 && chunks * 16 * (group / hpt) >= share * T;
+    };
+    const int hpt = fills(3, 1.0f) ? 3 : fills(2, 0.75f) ? 2 : 1;
+    const size_t lds = group_lds(span, p.max_chunks, T, group, hpt);
+    if (lds > (size_t)kGroupMaxLds) return 1;
+    const int per_cu = std::min(2048 / T, (int)(kGroupMaxLds / lds));
+    if (blocks > (int64_t)(per_cu > 1 ? 4 : 3) * p.cus * per_cu) return 1;
+    p.lmax = span;
+    return T == 1024 ? launch_group_hpt<1024>(p, hpt, lds, stream)
+                     : T == 512 ? launch_group_hpt<512>(p, hpt, lds, stream)
+                                : launch_group_hpt<256>(p, hpt, lds, stream);
+}
+
 int32_t attention_decode_impl(const int8_t* d_q, const float* d_qscale, int32_t rows, int32_t heads,
                               int32_t kv_heads, int32_t qk_dim, const int8_t* d_keys, const float* d_key_scales,
                               const int8_t* d_values, const float* d_value_scales, int32_t slots,
                               int32_t capacity, const int32_t* d_row_slot, const int32_t* d_row_first,
                               const int32_t* d_row_count, int32_t max_chunks, void* d_workspace,
                               size_t workspace_bytes, float* d_out, int8_t* d_q_out, float* d_qs_out,
-                              hipStream_t stream)
+                              int32_t max_count, hipStream_t stream)
 {
     clear_error();
     if (rows == 0) return NHIP_OK;
@@ -1509,13 +1881,17 @@ int32_t attention_decode_impl(const int8_t* d_q, const float* d_qscale, int32_t 
     const int head_blocks = (kv_heads + p.kv_per_block - 1) / p.kv_per_block;
     NHIP_REQUIRE(!d_q_out || (d_qs_out && max_chunks == 1 && head_blocks == 1),
                  "attention: a quantized output needs max_chunks 1 and all heads in one block");
+    p.cus = std::max(device_cus(), 1);
+    if (!d_q_out) {
+        rc = launch_group_attention(p, max_count, stream);
+        if (rc <= 0) return rc;
+    }
     if (!d_q_out && capacity <= kRowMaxCapacity) {  // every count <= capacity: one workgroup per (row, head)
         hipLaunchKernelGGL(decode_attention_row_kernel<kRowPlain>, dim3(rows, heads), dim3(row_threads(kRowPlain)), 0, stream,
                            ATTN_HEAD_ARGS(p, p.q, p.qscale), p);
         NHIP_CHECK_HIP(hipGetLastError());
         return NHIP_OK;
     }
-    p.cus = std::max(device_cus(), 1);
     p.cus_magic = p.cus == 1 ? 0u : 0xFFFFFFFFu / (uint32_t)p.cus + 1u;  // as magic(): exact for g < 2^16
     dim3 grid(max_chunks, rows, head_blocks);
     if (rows <= kPlacedRows) {  // placed units: whole rounds of p.cus workgroups
@@ -1567,7 +1943,7 @@ int32_t nhip_attention_decode_dev(const int8_t* d_q, const float* d_qscale, int3
 {
     return attention_decode_impl(d_q, d_qscale, rows, heads, kv_heads, qk_dim, d_keys, d_key_scales, d_values,
                                  d_value_scales, slots, capacity, d_row_slot, d_row_first, d_row_count, max_chunks,
-                                 d_workspace, workspace_bytes, d_out, nullptr, nullptr, as_stream(stream));
+                                 d_workspace, workspace_bytes, d_out, nullptr, nullptr, 0, as_stream(stream));
 }
 
 int32_t nhip_attention_decode_noalloc_dev(const int8_t* d_q, const float* d_qscale, int32_t rows, int32_t heads,
@@ -1594,7 +1970,7 @@ int32_t nhip_attention_decode_noalloc_dev(const int8_t* d_q, const float* d_qsca
     if (rc) return rc;
     return attention_decode_impl(d_q, d_qscale, rows, heads, kv_heads, qk_dim, d_keys, d_key_scales, d_values,
                                  d_value_scales, slots, capacity, d_row_slot, d_row_first, d_row_count, max_chunks, ws,
-                                 kAttentionScratchBytes, d_out, nullptr, nullptr, as_stream(stream));
+                                 kAttentionScratchBytes, d_out, nullptr, nullptr, 0, as_stream(stream));
 }
 
 }  // extern "C"

@@ -126,14 +126,15 @@ struct TileMatmul {
 int32_t launch_gemm_cq(WeightFormat fmt, const TileMatmul& p, bool special, hipStream_t stream);
 // Ragged decode attention (attention_decode.hip); with d_q_out the output
 // rows are also quantized (QuantizeInt8 per row), which needs max_chunks 1
-// and every head in one block.
+// and every head in one block.  max_count bounds the rows' counts (0: only the
+// capacity does).
 int32_t attention_decode_impl(const int8_t* d_q, const float* d_qscale, int32_t rows, int32_t heads,
                               int32_t kv_heads, int32_t qk_dim, const int8_t* d_keys, const float* d_key_scales,
                               const int8_t* d_values, const float* d_value_scales, int32_t slots,
                               int32_t capacity, const int32_t* d_row_slot, const int32_t* d_row_first,
                               const int32_t* d_row_count, int32_t max_chunks, void* d_workspace,
                               size_t workspace_bytes, float* d_out, int8_t* d_q_out, float* d_qs_out,
-                              hipStream_t stream);
+                              int32_t max_count, hipStream_t stream);
 // Decode matmul (1..4 tokens, literal int8 format, all rows) whose int8
 // activation rows are computed in the kernel's prologue from fp32 inputs
 // (gemv.hip): kProNorm = x (+ delta) -> RMSNorm * gain -> QuantizeInt8,

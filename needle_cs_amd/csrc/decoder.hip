@@ -915,7 +915,7 @@ int32_t enqueue_forward(nhip_decoder* m, int rows, const HeadPlan& hp, bool mask
             rc = attention_decode_impl(m->qh, m->qhs, rows, H, KV, 64, pp.keys, pp.key_scales, pp.values,
                                        pp.value_scales, D.slots, D.capacity, pp.slots, in_first(m, m->d_in),
                                        in_count(m, m->d_in), D.max_chunks, m->attn_ws, m->attn_ws_bytes, m->att,
-                                       attn_quant ? m->q8 : nullptr, attn_quant ? m->qs : nullptr, s);
+                                       attn_quant ? m->q8 : nullptr, attn_quant ? m->qs : nullptr, 0, s);
             if (rc) return rc;
         }
         rc = 1;

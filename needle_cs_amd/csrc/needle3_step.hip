@@ -37,12 +37,6 @@
 
 namespace nhip {
 
-int32_t attention_decode_impl(const int8_t* d_q, const float* d_qscale, int32_t rows, int32_t heads,
-                              int32_t kv_heads, int32_t qk_dim, const int8_t* d_keys, const float* d_key_scales,
-                              const int8_t* d_values, const float* d_value_scales, int32_t slots, int32_t capacity,
-                              const int32_t* d_row_slot, const int32_t* d_row_first, const int32_t* d_row_count,
-                              int32_t max_chunks, void* d_workspace, size_t workspace_bytes, float* d_out,
-                              int8_t* d_q_out, float* d_qs_out, hipStream_t stream);
 int32_t matmul_cq_split_internal(const DeviceWeights* w, const int8_t* values, const float* scales,
                                  const float* offsets, int32_t stride, int32_t tokens, float* const* ys,
                                  const int32_t* ldys, const int32_t* firsts, int32_t parts, hipStream_t stream);
@@ -1392,6 +1386,7 @@ struct nhip_ctx {
     uint64_t global_mask = 0;
     int slots = 0, capacity = 0, max_rows = 0, max_chunks = 0;
     int feed_rows = 0;  // rows of a FeedSlot step (>= max_rows); the scratch holds that many
+    int max_span = 0;   // of the current step's rows (steps that are not captured; 0: unknown)
     int in_stride = 0;  // of the current step's inputs: max_rows, or feed_rows for a longer step
     // weights
     nhip_weights* embedding = nullptr;
@@ -2073,7 +2068,7 @@ int32_t enqueue_step(nhip_ctx* c, int rows, int heads, int k, bool argmax, bool 
                 return rc;
             if ((rc = attention_decode_impl(c->q8, c->qs, rows, H, KV, c->qk, keys, kscale, values, vscale, c->slots,
                                             c->capacity, in(c, c->d_in, kInSlots), first, count, c->max_chunks,
-                                            c->attn_ws, c->attn_ws_bytes, c->att, nullptr, nullptr, s)))
+                                            c->attn_ws, c->attn_ws_bytes, c->att, nullptr, nullptr, c->max_span, s)))
                 return rc;
         }
         // the gate also moves the slots' Q/K/V frames on, after attention's
@@ -2240,6 +2235,8 @@ int32_t step_rows(nhip_ctx* c, const int32_t* tokens, const int32_t* row_slots, 
         }
         rs = rk + 1;
     }
+    c->max_span = 0;
+    for (int t = 0; rows > kMaxGraphRows && t < rows; t++) c->max_span = std::max(c->max_span, h[kInCount * R + t]);
     // the head runs once per distinct head row, in order of first mention;
     // repeated rows are copied out again
     for (int t = 0; t < rows; t++) h[kInHeadOf * R + t] = -1;
