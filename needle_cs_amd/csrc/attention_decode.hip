@@ -102,6 +102,10 @@ struct DecodeAttnParams {
 
 }  // namespace
 
+// The longest span of a launch whose rows' counts max_count bounds (0: only the
+// capacity does).
+static int span_bound(int max_count, int capacity) { return max_count > 0 ? std::min(max_count, capacity) : capacity; }
+
 // Longest chunk of the plan: at most 32 positions below 16*max_chunks
 // positions, else ceil(capacity/max_chunks) rounded up to 4.
 int decode_attention_lmax(int capacity, int max_chunks)
@@ -897,7 +901,7 @@ __global__ __launch_bounds__(T) void group_attention_kernel(ATTN_HEAD_PARAMS, De
     }
 }
 
-// Whole-row attention for caches of at most kRowMaxCapacity positions: one
+// Whole-row attention for spans of at most kRowMaxCapacity positions: one
 // workgroup per (row, query head) runs every chunk of the row's plan and then
 // merges them itself, with the chunk kernel's per-chunk arithmetic and
 // decode_merge_kernel's merge, so the results are the same bits.  For short
@@ -1180,7 +1184,7 @@ __global__ __launch_bounds__(row_threads(MODE)) void decode_attention_row_kernel
     }
     float* dst = p.out + ((size_t)row * p.heads + h) * 64;
     const bool valid = (slot_in >= 0) & (slot_in < p.slots) & (first_in >= 0) & (count_in >= 1) &
-                       (count_in <= p.capacity - first_in);
+                       (count_in <= p.capacity - first_in) & (count_in <= kRowMaxCapacity);
     const int slot = valid ? slot_in : 0;
     const int first = valid ? first_in : 0;
     const int count = valid ? count_in : 1;
@@ -1650,9 +1654,9 @@ int32_t attention_decode_post_impl(const AttnPostInputs& in, int32_t rows, int32
                                    int8_t* d_keys, float* d_key_scales, int8_t* d_values, float* d_value_scales,
                                    int32_t slots, int32_t capacity, const int32_t* d_row_slot,
                                    const int32_t* d_row_first, const int32_t* d_row_count, int32_t max_chunks,
-                                   float* d_out, hipStream_t stream)
+                                   int32_t max_count, float* d_out, hipStream_t stream)
 {
-    if (rows < 1 || rows > kPostRows || capacity > kRowMaxCapacity) return 1;
+    if (rows < 1 || rows > kPostRows || span_bound(max_count, capacity) > kRowMaxCapacity) return 1;
     NHIP_REQUIRE(heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && slots > 0 && capacity > 0 && max_chunks >= 1,
                  "attention: bad shape");
     NHIP_REQUIRE(in.qkv && in.positions && in.rope_rows && d_keys && d_key_scales && d_values &&
@@ -1688,16 +1692,16 @@ int32_t attention_decode_post_impl(const AttnPostInputs& in, int32_t rows, int32
     return NHIP_OK;
 }
 
-bool attention_needle3_fused(int32_t capacity, int32_t v_dim) { return capacity <= kRowMaxCapacity && v_dim == 64; }
+bool attention_needle3_fused(int32_t span, int32_t v_dim) { return span <= kRowMaxCapacity && v_dim == 64; }
 
 int32_t attention_decode_needle3_impl(const Needle3AttnInputs& in, int32_t rows, int32_t heads, int32_t kv_heads,
                                       int32_t qk_dim, int32_t v_dim, int8_t* d_keys, float* d_key_scales,
                                       int8_t* d_values, float* d_value_scales, int32_t slots, int32_t capacity,
                                       const int32_t* d_row_slot, const int32_t* d_row_pos,
                                       const int32_t* d_row_first, const int32_t* d_row_count, int32_t max_chunks,
-                                      float* d_out, hipStream_t stream)
+                                      int32_t max_count, float* d_out, hipStream_t stream)
 {
-    if (rows < 1 || !attention_needle3_fused(capacity, v_dim)) return 1;
+    if (rows < 1 || !attention_needle3_fused(span_bound(max_count, capacity), v_dim)) return 1;
     NHIP_REQUIRE(heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && slots > 0 && capacity > 0 && max_chunks >= 1,
                  "attention: bad shape");
     NHIP_REQUIRE(qk_dim == 48 || qk_dim == 64, "attention: qk_dim must be 48 or 64 (got %d)", qk_dim);
@@ -1792,10 +1796,10 @@ int32_t launch_group_hpt(const DecodeAttnParams& p, int hpt, size_t lds, hipStre
 int32_t launch_group_attention(DecodeAttnParams p, int32_t max_count, hipStream_t stream)
 {
     const int group = p.heads / p.kv_heads;
-    const int span = max_count > 0 ? std::min(max_count, p.capacity) : p.capacity;
+    const int span = span_bound(max_count, p.capacity);
     const int chunks = std::min(p.max_chunks, std::max(span / 16, 1));
     if (p.rows <= kPlacedRows && p.rows * chunks <= 2560) return 1;
-    if (p.capacity <= kRowMaxCapacity && (group == 1 || (int64_t)p.rows * p.heads < 1024)) return 1;
+    if (span <= kRowMaxCapacity && (group == 1 || (int64_t)p.rows * p.heads < 1024)) return 1;
     const int64_t blocks = (int64_t)p.rows * p.kv_heads;
     const bool own = p.rows < 8 * (int64_t)p.slots;  // few rows a slot
     if (own && (group == 1 || span > 1024 || blocks > 1024)) return 1;
@@ -1886,7 +1890,7 @@ int32_t attention_decode_impl(const int8_t* d_q, const float* d_qscale, int32_t 
         rc = launch_group_attention(p, max_count, stream);
         if (rc <= 0) return rc;
     }
-    if (!d_q_out && capacity <= kRowMaxCapacity) {  // every count <= capacity: one workgroup per (row, head)
+    if (!d_q_out && span_bound(max_count, capacity) <= kRowMaxCapacity) {  // one workgroup per (row, head)
         hipLaunchKernelGGL(decode_attention_row_kernel<kRowPlain>, dim3(rows, heads), dim3(row_threads(kRowPlain)), 0, stream,
                            ATTN_HEAD_ARGS(p, p.q, p.qscale), p);
         NHIP_CHECK_HIP(hipGetLastError());

@@ -192,7 +192,8 @@ constexpr int kFusedPrologueMaxTiles = 512;
 // QuantizeInt8, and each row's key and value write to the cache at its
 // position (qk 64).  Rows of the batch that write positions of another row's
 // span are read from the launch's own results.  Returns 1 without launching
-// when it does not apply: more than 4 rows or caches over 512 positions.
+// when it does not apply: more than 4 rows or spans over 512 positions (of the
+// capacity, or of max_count where that bounds the rows' counts).
 struct AttnPostInputs {
     const float* qkv;          // [rows][(heads + 2 kv_heads) * 64]
     const int32_t* positions;  // [rows]
@@ -201,7 +202,7 @@ struct AttnPostInputs {
 int32_t attention_decode_post_impl(const AttnPostInputs& in, int32_t rows, int32_t heads, int32_t kv_heads,
                                    int8_t* d_keys, float* d_key_scales, int8_t* d_values, float* d_value_scales,
                                    int32_t slots, int32_t capacity, const int32_t* d_row_slot,
-                                   const int32_t* d_row_first, const int32_t* d_row_count, int32_t max_chunks,
+                                   const int32_t* d_row_first, const int32_t* d_row_count, int32_t max_chunks, int32_t max_count,
                                    float* d_out, hipStream_t stream);
 // Needle 3's attention inputs and decode attention in one launch (the
 // whole-row kernel's Needle 3 form), for steps whose rows are one per slot
@@ -285,14 +286,14 @@ struct Needle3AttnInputs {
     const float* b_res;  // [16]
     Needle3Proj proj;
 };
-// Whether attention_decode_needle3_impl takes a step (caches of at most 512
+// Whether attention_decode_needle3_impl takes a step (spans of at most 512
 // positions, value heads of 64).
-bool attention_needle3_fused(int32_t capacity, int32_t v_dim);
+bool attention_needle3_fused(int32_t span, int32_t v_dim);
 int32_t attention_decode_needle3_impl(const Needle3AttnInputs& in, int32_t rows, int32_t heads, int32_t kv_heads,
                                       int32_t qk_dim, int32_t v_dim, int8_t* d_keys, float* d_key_scales,
                                       int8_t* d_values, float* d_value_scales, int32_t slots, int32_t capacity,
                                       const int32_t* d_row_slot, const int32_t* d_row_pos,
-                                      const int32_t* d_row_first, const int32_t* d_row_count, int32_t max_chunks,
+                                      const int32_t* d_row_first, const int32_t* d_row_count, int32_t max_chunks, int32_t max_count,
                                       float* d_out, hipStream_t stream);
 // nhip_needle3_attention_inputs_dev; with_history false leaves the slots'
 // Q/K/V frames to the caller, which moves them on after every row of the

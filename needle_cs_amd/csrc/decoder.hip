@@ -732,6 +732,7 @@ struct HeadPlan {
 // device memory the host refreshes before each launch.
 struct StepGraph {
     int rows;
+    int max_span;
     HeadPlan head;
     hipGraphExec_t exec;
 };
@@ -739,6 +740,7 @@ struct StepGraph {
 struct nhip_decoder {
     nhip_decoder_dims dims{};
     int qkv_n = 0;
+    int max_span = 0;  // bounds the staged rows' counts: kShortSpan or the capacity
     std::vector<nhip_weights*> wqkv, wo, wgu, wd;
     nhip_weights* wlm = nullptr;
     std::vector<float*> attn_norm, ffn_norm;
@@ -906,7 +908,7 @@ int32_t enqueue_forward(nhip_decoder* m, int rows, const HeadPlan& hp, bool mask
             const AttnPostInputs in{m->qkv, pp.positions, in_rope(m, m->d_in)};
             rc = attention_decode_post_impl(in, rows, H, KV, pp.keys, pp.key_scales, pp.values, pp.value_scales,
                                             D.slots, D.capacity, pp.slots, in_first(m, m->d_in),
-                                            in_count(m, m->d_in), D.max_chunks, m->att, s);
+                                            in_count(m, m->d_in), D.max_chunks, m->max_span, m->att, s);
             if (rc < 0) return rc;
         }
         if (rc) {
@@ -915,7 +917,7 @@ int32_t enqueue_forward(nhip_decoder* m, int rows, const HeadPlan& hp, bool mask
             rc = attention_decode_impl(m->qh, m->qhs, rows, H, KV, 64, pp.keys, pp.key_scales, pp.values,
                                        pp.value_scales, D.slots, D.capacity, pp.slots, in_first(m, m->d_in),
                                        in_count(m, m->d_in), D.max_chunks, m->attn_ws, m->attn_ws_bytes, m->att,
-                                       attn_quant ? m->q8 : nullptr, attn_quant ? m->qs : nullptr, 0, s);
+                                       attn_quant ? m->q8 : nullptr, attn_quant ? m->qs : nullptr, m->max_span, s);
             if (rc) return rc;
         }
         rc = 1;
@@ -1004,10 +1006,15 @@ int32_t enqueue_forward(nhip_decoder* m, int rows, const HeadPlan& hp, bool mask
     return NHIP_OK;
 }
 
+// Steps whose spans are at most this take the attention kernels of short
+// caches, whatever the capacity.
+constexpr int kShortSpan = 512;
+
 int32_t stage_inputs(nhip_decoder* m, const int32_t* tokens, const int32_t* slots, const int32_t* positions,
                      int rows, const int32_t* head_rows = nullptr, int heads = 0)
 {
     const nhip_decoder_dims& D = m->dims;
+    int span = 0;
     for (int r = 0; r < rows; r++) {
         NHIP_REQUIRE(tokens[r] >= 0 && tokens[r] < D.vocab, "token %d out of range", tokens[r]);
         NHIP_REQUIRE(slots[r] >= 0 && slots[r] < D.slots, "slot %d out of range", slots[r]);
@@ -1018,10 +1025,12 @@ int32_t stage_inputs(nhip_decoder* m, const int32_t* tokens, const int32_t* slot
         in_positions(m, m->h_in)[r] = positions[r];
         in_first(m, m->h_in)[r] = 0;
         in_count(m, m->h_in)[r] = positions[r] + 1;
+        span = std::max(span, positions[r] + 1);
         float* rope = in_rope(m, m->h_in) + (size_t)r * 64;
         std::memcpy(rope, m->rope_cos_h.data() + (size_t)positions[r] * 32, 32 * sizeof(float));
         std::memcpy(rope + 32, m->rope_sin_h.data() + (size_t)positions[r] * 32, 32 * sizeof(float));
     }
+    m->max_span = span <= kShortSpan ? std::min(kShortSpan, D.capacity) : D.capacity;
     for (int i = 0; i < heads; i++) {
         NHIP_REQUIRE(head_rows[i] >= 0 && head_rows[i] < rows, "head row %d outside [0, %d)", head_rows[i], rows);
         in_heads(m, m->h_in)[i] = head_rows[i];
@@ -1050,7 +1059,7 @@ int32_t run_staged(nhip_decoder* m, int rows, const HeadPlan& hp, bool use_graph
     if (use_graph) {
         hipGraphExec_t exec = nullptr;
         for (const StepGraph& g : m->graphs)
-            if (g.rows == rows && g.head == hp) exec = g.exec;
+            if (g.rows == rows && g.max_span == m->max_span && g.head == hp) exec = g.exec;
         if (!exec) {
             if (m->graphs.size() >= kMaxGraphs) {  // drop the oldest
                 NHIP_CHECK_HIP(hipStreamSynchronize(m->stream));
@@ -1069,7 +1078,7 @@ int32_t run_staged(nhip_decoder* m, int rows, const HeadPlan& hp, bool use_graph
             e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
             (void)hipGraphDestroy(g);
             NHIP_CHECK_HIP(e);
-            m->graphs.push_back(StepGraph{rows, hp, exec});
+            m->graphs.push_back(StepGraph{rows, m->max_span, hp, exec});
         }
         NHIP_CHECK_HIP(hipGraphLaunch(exec, m->stream));
     } else {

@@ -1386,7 +1386,7 @@ struct nhip_ctx {
     uint64_t global_mask = 0;
     int slots = 0, capacity = 0, max_rows = 0, max_chunks = 0;
     int feed_rows = 0;  // rows of a FeedSlot step (>= max_rows); the scratch holds that many
-    int max_span = 0;   // of the current step's rows (steps that are not captured; 0: unknown)
+    int max_span = 0;   // bounds the current step's counts: kShortSpan or the capacity for steps that are captured
     int in_stride = 0;  // of the current step's inputs: max_rows, or feed_rows for a longer step
     // weights
     nhip_weights* embedding = nullptr;
@@ -1428,6 +1428,7 @@ struct nhip_ctx {
     struct Graph {
         int rows, heads, k;
         bool argmax, single_runs;
+        int max_span;
         hipGraphExec_t exec;
     };
     std::vector<Graph> graphs;  // captured steps, by their shape
@@ -1897,7 +1898,7 @@ int32_t enqueue_step(nhip_ctx* c, int rows, int heads, int k, bool argmax, bool 
     // steps whose rows are one per slot run the attention in one launch
     // (attention_decode_needle3_impl), which then also forms Sinkhorn4x4 of
     // the mix kernel's residual-mix logits
-    const bool sink_in_attention = single_runs && attention_needle3_fused(c->capacity, c->vd);
+    const bool sink_in_attention = single_runs && attention_needle3_fused(c->max_span, c->vd);
     auto site_of = [&](int l) -> const N3Site* {
         for (int k2 = 0; k2 < c->site_count; k2++)
             if (c->sites[k2] == l) return &c->site[k2];
@@ -2055,7 +2056,8 @@ int32_t enqueue_step(nhip_ctx* c, int rows, int heads, int k, bool argmax, bool 
             }
             fused = attention_decode_needle3_impl(n3in, rows, H, KV, c->qk, c->vd, keys, kscale, values, vscale,
                                                   c->slots, c->capacity, in(c, c->d_in, kInSlots),
-                                                  in(c, c->d_in, kInPos), first, count, c->max_chunks, c->att, s);
+                                                  in(c, c->d_in, kInPos), first, count, c->max_chunks, c->max_span,
+                                                  c->att, s);
             if (fused < 0) return fused;
             NHIP_REQUIRE(fused == 0 || !sink_in_attention, "attention launch refused a step it takes");
         }
@@ -2122,12 +2124,17 @@ int32_t enqueue_step(nhip_ctx* c, int rows, int heads, int k, bool argmax, bool 
 }
 
 // Steps of up to kMaxGraphRows rows replay a graph captured on first use for
-// their (rows, heads, k, argmax): every per-step input lives in device
+// their (rows, heads, k, argmax, one row per slot, span bound): every per-step input lives in device
 // arrays uploaded before the launch, so the captured kernels and arguments
 // stay valid.  NHIP_ENGINE_GRAPHS=0 launches every step eagerly (for kernel
 // tracers).
 constexpr int kMaxGraphRows = 16;
 constexpr size_t kMaxGraphs = 64;
+// Steps whose spans are at most this run their attention in one launch with its
+// inputs (attention_needle3_fused), whatever the capacity: 16 slots of a
+// 1024-position context at positions 60-68, 8 steps: 8.76 ms, 10.47 with the
+// attention inputs, the chunk kernel and its merge in launches of their own.
+constexpr int kShortSpan = 512;
 
 int32_t run_step(nhip_ctx* c, int rows, int heads, int k, bool argmax, bool single_runs)
 {
@@ -2138,7 +2145,8 @@ int32_t run_step(nhip_ctx* c, int rows, int heads, int k, bool argmax, bool sing
     if (!graphs_enabled || rows > kMaxGraphRows) return enqueue_step(c, rows, heads, k, argmax, single_runs);
     hipGraphExec_t exec = nullptr;
     for (const nhip_ctx::Graph& g : c->graphs)
-        if (g.rows == rows && g.heads == heads && g.k == k && g.argmax == argmax && g.single_runs == single_runs)
+        if (g.rows == rows && g.heads == heads && g.k == k && g.argmax == argmax && g.single_runs == single_runs &&
+            g.max_span == c->max_span)
             exec = g.exec;
     if (!exec) {
         if (c->graphs.size() >= kMaxGraphs) {  // drop the oldest
@@ -2158,7 +2166,7 @@ int32_t run_step(nhip_ctx* c, int rows, int heads, int k, bool argmax, bool sing
         e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         NHIP_CHECK_HIP(e);
-        c->graphs.push_back(nhip_ctx::Graph{rows, heads, k, argmax, single_runs, exec});
+        c->graphs.push_back(nhip_ctx::Graph{rows, heads, k, argmax, single_runs, c->max_span, exec});
     }
     NHIP_CHECK_HIP(hipGraphLaunch(exec, c->stream_h));
     return NHIP_OK;
@@ -2236,7 +2244,8 @@ int32_t step_rows(nhip_ctx* c, const int32_t* tokens, const int32_t* row_slots, 
         rs = rk + 1;
     }
     c->max_span = 0;
-    for (int t = 0; rows > kMaxGraphRows && t < rows; t++) c->max_span = std::max(c->max_span, h[kInCount * R + t]);
+    for (int t = 0; t < rows; t++) c->max_span = std::max(c->max_span, h[kInCount * R + t]);
+    if (rows <= kMaxGraphRows) c->max_span = c->max_span <= kShortSpan ? std::min(kShortSpan, c->capacity) : c->capacity;
     // the head runs once per distinct head row, in order of first mention;
     // repeated rows are copied out again
     for (int t = 0; t < rows; t++) h[kInHeadOf * R + t] = -1;
