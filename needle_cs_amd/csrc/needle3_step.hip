@@ -1345,6 +1345,57 @@ __global__ __launch_bounds__(kThreads) void n3_tail_kernel(const float* h_proj, 
     prepare_row_fake(res, dim, 4, a.act, a.stride, head, inverse, round, scale);
 }
 
+// ------------------------------------------------------- slot state --
+
+// A slot's histories in one launch, block column y < layers layer y's Q/K/V
+// frames, the others site y - layers' engram frames: to[...] = from[...], or
+// zeros where from is null.  The slots' frames are 2 * all (hist) and eh floats
+// apart, layers and sites `slots` of those; multiples of 4 floats (the widths
+// are multiples of 16).  Mark, rewind and reset were a copy or a fill per layer
+// and site (25 at Needle 3's geometry): a rewind 94 -> 12 us, a reset 81 -> 12,
+// a copy of a 60-position slot 362 -> 19.
+struct SlotState {
+    float *hist, *engram;
+};
+constexpr int kSlotBlock = 256;
+__global__ __launch_bounds__(kSlotBlock) void n3_slot_state_kernel(SlotState to, SlotState from, int to_slot,
+                                                                   int from_slot, int slots, int layers, int hist,
+                                                                   int eh)
+{
+    const int y = blockIdx.y;
+    const bool qkv = y < layers;
+    const int n = qkv ? hist : eh;
+    const int i = 4 * ((int)blockIdx.x * kSlotBlock + (int)threadIdx.x);
+    if (i >= n) return;
+    const size_t at = (size_t)(qkv ? y : y - layers) * slots;
+    const float* src = qkv ? from.hist : from.engram;
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (src) v = *reinterpret_cast<const float4*>(src + (at + from_slot) * n + i);
+    *reinterpret_cast<float4*>((qkv ? to.hist : to.engram) + (at + to_slot) * n + i) = v;
+}
+
+// Slot src's first n cache positions to slot dst, every layer in one launch
+// (block column y): keys and values 16 bytes a thread, then the scales.
+__global__ __launch_bounds__(kSlotBlock) void n3_slot_cache_kernel(int8_t* keys, int8_t* values, float* kscale,
+                                                                   float* vscale, int dst, int src, int slots,
+                                                                   int capacity, int n, int kw, int vw, int kv)
+{
+    const size_t cd = ((size_t)blockIdx.y * slots + dst) * capacity, cs = ((size_t)blockIdx.y * slots + src) * capacity;
+    const int stride = gridDim.x * kSlotBlock, u = blockIdx.x * kSlotBlock + threadIdx.x;
+    const size_t k16 = (size_t)n * kw / 16, v16 = (size_t)n * vw / 16, sc = (size_t)n * kv;
+    const auto copy16 = [&](int8_t* base, int width, size_t count) {
+        const uint4* from = reinterpret_cast<const uint4*>(base + cs * width);
+        uint4* to = reinterpret_cast<uint4*>(base + cd * width);
+        for (size_t i = u; i < count; i += stride) to[i] = from[i];
+    };
+    copy16(keys, kw, k16);
+    copy16(values, vw, v16);
+    for (size_t i = u; i < sc; i += stride) {
+        kscale[cd * kv + i] = kscale[cs * kv + i];
+        vscale[cd * kv + i] = vscale[cs * kv + i];
+    }
+}
+
 }  // namespace
 }  // namespace nhip
 
@@ -2172,29 +2223,25 @@ int32_t run_step(nhip_ctx* c, int rows, int heads, int k, bool argmax, bool sing
     return NHIP_OK;
 }
 
+// One launch over a slot's histories (n3_slot_state_kernel); from.hist null: zeros.
+int32_t slot_state(nhip_ctx* c, SlotState to, SlotState from, int to_slot, int from_slot)
+{
+    const int hist = 2 * (c->heads * c->qk + c->kv * c->qk + c->kv * c->vd), eh = kEngramHistory * c->dim;
+    const int widest = c->site_count > 0 ? std::max(hist, eh) : hist;
+    hipLaunchKernelGGL(n3_slot_state_kernel, dim3((widest / 4 + kSlotBlock - 1) / kSlotBlock, c->layers + c->site_count),
+                       dim3(kSlotBlock), 0, c->stream_h, to, from, to_slot, from_slot, c->slots, c->layers, hist, eh);
+    NHIP_CHECK_HIP(hipGetLastError());
+    return NHIP_OK;
+}
+
 // The live histories of a slot (convolution frames of every layer, engram
 // frames of every site) to or from its snapshot; MarkView / RewindView
 // (Engine.cs:2235-2255) with the rewind restoring eagerly.
 int32_t snapshot_slot(nhip_ctx* c, int slot, bool to_snapshot)
 {
-    const size_t all = (size_t)c->heads * c->qk + (size_t)c->kv * c->qk + (size_t)c->kv * c->vd;
-    int32_t rc;
-    for (int l = 0; l < c->layers; l++) {
-        const size_t o = ((size_t)l * c->slots + slot) * 2 * all;
-        float* live = c->qkv_hist + o;
-        float* snap = c->snap_qkv + o;
-        if ((rc = nhip_copy_dev(to_snapshot ? snap : live, to_snapshot ? live : snap, sizeof(float) * 2 * all,
-                                c->stream_h)))
-            return rc;
-    }
-    const size_t eh = (size_t)kEngramHistory * c->dim;
-    for (int k = 0; k < c->site_count; k++) {
-        const size_t o = ((size_t)k * c->slots + slot) * eh;
-        float* live = c->engram_hist + o;
-        float* snap = c->snap_engram + o;
-        if ((rc = nhip_copy_dev(to_snapshot ? snap : live, to_snapshot ? live : snap, sizeof(float) * eh, c->stream_h)))
-            return rc;
-    }
+    const SlotState live{c->qkv_hist, c->engram_hist}, snap{c->snap_qkv, c->snap_engram};
+    const int32_t rc = slot_state(c, to_snapshot ? snap : live, to_snapshot ? live : snap, slot, slot);
+    if (rc) return rc;
     for (int i = 0; i < 2; i++) {
         if (to_snapshot) c->snap_prev[2 * slot + i] = c->prev[2 * slot + i];
         else c->prev[2 * slot + i] = c->snap_prev[2 * slot + i];
@@ -2444,14 +2491,8 @@ int32_t nhip_slot_reset(nhip_ctx* c, int32_t slot)
 {
     clear_error();
     NHIP_REQUIRE(c && slot >= 0 && slot < c->slots, "slot %d outside the context's slots", slot);
-    const size_t all = (size_t)c->heads * c->qk + (size_t)c->kv * c->qk + (size_t)c->kv * c->vd;
-    for (int l = 0; l < c->layers; l++)
-        NHIP_CHECK_HIP(hipMemsetAsync(c->qkv_hist + ((size_t)l * c->slots + slot) * 2 * all, 0, sizeof(float) * 2 * all,
-                                      c->stream_h));
-    const size_t eh = (size_t)kEngramHistory * c->dim;
-    for (int k = 0; k < c->site_count; k++)
-        NHIP_CHECK_HIP(
-            hipMemsetAsync(c->engram_hist + ((size_t)k * c->slots + slot) * eh, 0, sizeof(float) * eh, c->stream_h));
+    const int32_t rc = slot_state(c, SlotState{c->qkv_hist, c->engram_hist}, SlotState{}, slot, slot);
+    if (rc) return rc;
     NHIP_CHECK_HIP(hipStreamSynchronize(c->stream_h));
     c->prev[2 * slot] = c->prev[2 * slot + 1] = 0;
     c->len[slot] = 0;
@@ -2493,27 +2534,16 @@ int32_t nhip_slot_copy(nhip_ctx* c, int32_t dst, int32_t src)
     NHIP_REQUIRE(c && dst >= 0 && dst < c->slots && src >= 0 && src < c->slots, "slots %d <- %d outside [0, %d)", dst,
                  src, c ? c->slots : 0);
     if (dst == src) return NHIP_OK;
-    const size_t qw = (size_t)c->heads * c->qk, kw = (size_t)c->kv * c->qk, vw = (size_t)c->kv * c->vd,
-                 all = qw + kw + vw, n = (size_t)c->len[src], KV = c->kv;
+    const int kw = c->kv * c->qk, vw = c->kv * c->vd, n = c->len[src];
     hipStream_t s = c->stream_h;
     int32_t rc;
-    for (int l = 0; l < c->layers; l++) {
-        const size_t cs = ((size_t)l * c->slots + src) * c->capacity, cd = ((size_t)l * c->slots + dst) * c->capacity;
-        const size_t hs = ((size_t)l * c->slots + src) * 2 * all, hd = ((size_t)l * c->slots + dst) * 2 * all;
-        if ((rc = nhip_copy_dev(c->keys + cd * kw, c->keys + cs * kw, n * kw, s)) ||
-            (rc = nhip_copy_dev(c->values + cd * vw, c->values + cs * vw, n * vw, s)) ||
-            (rc = nhip_copy_dev(c->key_scales + cd * KV, c->key_scales + cs * KV, n * KV * sizeof(float), s)) ||
-            (rc = nhip_copy_dev(c->value_scales + cd * KV, c->value_scales + cs * KV, n * KV * sizeof(float), s)) ||
-            (rc = nhip_copy_dev(c->qkv_hist + hd, c->qkv_hist + hs, 2 * all * sizeof(float), s)) ||
-            (rc = nhip_copy_dev(c->snap_qkv + hd, c->snap_qkv + hs, 2 * all * sizeof(float), s)))
-            return rc;
-    }
-    const size_t eh = (size_t)kEngramHistory * c->dim;
-    for (int k = 0; k < c->site_count; k++) {
-        const size_t os = ((size_t)k * c->slots + src) * eh, od = ((size_t)k * c->slots + dst) * eh;
-        if ((rc = nhip_copy_dev(c->engram_hist + od, c->engram_hist + os, eh * sizeof(float), s)) ||
-            (rc = nhip_copy_dev(c->snap_engram + od, c->snap_engram + os, eh * sizeof(float), s)))
-            return rc;
+    const SlotState live{c->qkv_hist, c->engram_hist}, snap{c->snap_qkv, c->snap_engram};
+    if ((rc = slot_state(c, live, live, dst, src)) || (rc = slot_state(c, snap, snap, dst, src))) return rc;
+    if (n > 0) {
+        const int blocks = (int)std::min<size_t>(((size_t)n * vw / 16 + kSlotBlock - 1) / kSlotBlock, 64);
+        hipLaunchKernelGGL(n3_slot_cache_kernel, dim3(blocks, c->layers), dim3(kSlotBlock), 0, s, c->keys, c->values,
+                           c->key_scales, c->value_scales, dst, src, c->slots, c->capacity, n, kw, vw, c->kv);
+        NHIP_CHECK_HIP(hipGetLastError());
     }
     NHIP_CHECK_HIP(hipStreamSynchronize(s));
     for (int i = 0; i < 2; i++) {
