@@ -206,7 +206,7 @@ int32_t attention_decode_post_impl(const AttnPostInputs& in, int32_t rows, int32
                                    float* d_out, hipStream_t stream);
 // Needle 3's attention inputs and decode attention in one launch (the
 // whole-row kernel's Needle 3 form), for steps whose rows are one per slot
-// and caches of at most 512 positions: each (row, query head) workgroup forms
+// and spans of at most 512 positions: each (row, query head) workgroup forms
 // its query head, and the row's key and value heads, from the raw Q/K/V
 // projections as needle3_attention_inputs_impl does (three-tap convolution
 // over the slot's two previous frames, ZeroCenteredRms and RoPE of the query
@@ -214,7 +214,7 @@ int32_t attention_decode_post_impl(const AttnPostInputs& in, int32_t rows, int32
 // value in place of the cache at the row's position, and the group's first
 // query head writes that key and value to the cache.  The slots' frames are
 // left for the caller to move on.  Returns 1 without launching when it does
-// not apply (caches over 512 positions, value heads other than 64).
+// not apply (spans over 512 positions, value heads other than 64).
 // Prepared activations (Quant.Activations): row t's values at values + t * cols,
 // its group scales and offsets at scales / offsets + t * stride.
 struct Act {

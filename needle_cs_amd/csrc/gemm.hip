@@ -198,22 +198,28 @@ __device__ __forceinline__ void gemm_i8_body(const GemmParams& p)
         }
     };
 
-    // pipeline: stage st+1's loads are in flight while stage st is
-    // multiplied (the last iteration reloads the last stage, unused)
-    WStage<TPW> wcur, wnext;
-    load_a(0, 0);
-    load_w(wcur, 0);
-    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-    __syncthreads();
-    for (int st = 0; st < stages; st++) {
-        const int buf = st & 1;
+    // pipeline: stage st+1's loads are in flight while stage st is multiplied
+    // (the last iteration reloads the last stage, unused).  Two register sets
+    // by turns: copied from one to the other, the copies were scheduled into
+    // the stage, and with them the wait for the loads (128 x 4096 x 1024 exact
+    // 11.4 -> 9.0 us, 128 x 1024 x 1024 4.2 -> 3.8, 512 x 2048 x 8192 fused
+    // 31.5 -> 29.5)
+    WStage<TPW> w0, w1;
+    auto step = [&](const WStage<TPW>& cur, WStage<TPW>& next, int buf, int st) {
         const int nst = min(st + 1, stages - 1);
         load_a(buf ^ 1, nst);  // that buffer was last read in the previous stage, before the barrier
-        load_w(wnext, nst);
-        compute(wcur, buf, st);
-        wcur = wnext;
+        load_w(next, nst);
+        compute(cur, buf, st);
         __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);  // this wave's LDS writes of the next stage have landed
         __syncthreads();
+    };
+    load_a(0, 0);
+    load_w(w0, 0);
+    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+    __syncthreads();
+    for (int st = 0; st < stages; st += 2) {
+        step(w0, w1, 0, st);
+        if (st + 1 < stages) step(w1, w0, 1, st + 1);
     }
 
 #pragma unroll
@@ -257,11 +263,12 @@ int32_t launch(const GemmParams& p, bool special, hipStream_t stream)
         return (int64_t)((tiles + 4 * tpw - 1) / (4 * tpw)) * ((p.tokens + 16 * ti - 1) / (16 * ti));
     };
     // The largest tile that leaves two workgroups for every CU.  Measured for
-    // 64 x 128 / 32 x 64 / 16 x 64, exact: 512 x 2048 x 8192 38.7 / 41.8 / - us
-    // (512 workgroups of 64 x 128); 512 x 2048 x 4096 27.2 / 22.8 / 28.3 (256);
-    // 128 x 1024 x 8192 14.4 / 8.1 / 8.6 (128; 512 of 32 x 64); 256 x 1024 x
-    // 3072 14.2 / 7.7 / 7.2 (384 of 32 x 64); 128 x 1024 x 1024 13.5 / 5.6 / 4.2;
-    // 128 x 4096 x 1024 43.7 / 15.6 / 11.5 (one chain of 128 groups a wave).
+    // 64 x 128 / 32 x 64 / 16 x 64, exact (before the two register sets):
+    // 512 x 2048 x 8192 38.7 / 41.8 / - us (512 workgroups of 64 x 128);
+    // 512 x 2048 x 4096 27.2 / 22.8 / 28.3 (256); 128 x 1024 x 8192 14.4 / 8.1 /
+    // 8.6 (128; 512 of 32 x 64); 256 x 1024 x 3072 14.2 / 7.7 / 7.2 (384 of
+    // 32 x 64); 128 x 1024 x 1024 13.5 / 5.6 / 4.2; 128 x 4096 x 1024 43.7 /
+    // 15.6 / 11.5 (one chain of 128 groups a wave).
     if (groups_of(4, 2) >= 512) return launch_tile<EXACT, 4, 2>(p, special, stream);
     if (groups_of(2, 1) >= 512) return launch_tile<EXACT, 2, 1>(p, special, stream);
     return launch_tile<EXACT, 1, 1>(p, special, stream);
