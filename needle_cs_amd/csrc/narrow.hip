@@ -340,7 +340,7 @@ int32_t launch_i8_narrow(const DeviceWeights* w, int32_t kind, const void* in, c
     if (rw != 4 && rw != 8) return 1;
     int waves = forced_waves ? forced_waves : (w->cols >= 2048 ? 8 : 4);
     if (kind == kProNorm || (waves == 8 && w->cols < 2048)) waves = 4;
-    NHIP_REQUIRE(in && y && ldy >= w->rows, "narrow matmul: null input/output or ldy %d below %d rows", ldy, w->rows);
+    NHIP_REQUIRE(in && y && ldy >= row_end, "narrow matmul: null input/output or ldy %d below row %d", ldy, row_end);
     NHIP_REQUIRE(kind != 0 || qscale, "narrow matmul: int8 rows without scales");
     NHIP_REQUIRE(kind != kProNorm || gain, "narrow matmul: RMSNorm without a gain");
     const int K = w->cols;

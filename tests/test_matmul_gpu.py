@@ -464,3 +464,16 @@ def test_int8_narrow_decode_bit_exact(hip, orc, tokens, rows, cols, r0, r1):
     want = np.full((tokens, rows + 3), SENTINEL, dtype=np.float32)
     orc.matmul_rows_i8(w, scales, q, qs, tokens, want, rows + 3, r0, r1)
     assert np.array_equal(y.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("tokens", [1, 3, 4])
+def test_narrow_output_stride_of_the_row_range(hip, orc, tokens):
+    """A row range needs an output stride of its last row only, not of the
+    matrix: the narrow kernel's shape (K 1024) too."""
+    rows, cols, r0, r1 = 96, 1024, 5, 40
+    w, scales, x, q, qs = int8_case(orc, 900 + tokens, rows, cols, tokens)
+    weights = hip.Weights.int8(w, scales)
+    want = np.full((tokens, r1), SENTINEL, dtype=np.float32)
+    orc.matmul_rows_i8(w, scales, q, qs, tokens, want, r1, r0, r1)
+    y = run_i8(hip, weights, q, qs, tokens, r1, r0, r1)
+    assert np.array_equal(y.view(np.uint32), want.view(np.uint32))
