@@ -207,7 +207,8 @@ int32_t nhip_prepare_dev(const float* d_x, int32_t tokens, int32_t cols, int32_t
 
 /* y[t*ldy+n] = sum_g (h(scale[n][g]) * qscale[t]) * dot_g(w[n], q[t]) for
  * n in [row_start,row_end), t < tokens, in Scalar.MatMulRows' order
- * (Scalar.cs:160-189).  Literal int8 weights. */
+ * (Scalar.cs:160-189).  Literal int8 weights.  Past 16 tokens a
+ * 16-byte aligned d_q takes a faster kernel. */
 int32_t nhip_matmul_i8_dev(const nhip_weights* w, const int8_t* d_q, const float* d_qscale,
                            int32_t tokens, float* d_y, int32_t ldy, int32_t row_start,
                            int32_t row_end, void* stream);
@@ -225,13 +226,15 @@ int32_t nhip_read_stream_dev(const void* d_src, size_t bytes, uint32_t* d_sink, 
  * and scaled once, y = acc * qscale[t] -- two VALU operations per (token,
  * row, group) instead of the reference's four, so the fp32 outputs agree with
  * Scalar.MatMulRows to 1e-4 of RMS(y), not bit for bit.  For prefill
- * throughput; nhip_matmul_i8_dev stays bit-exact for every token count. */
+ * throughput; nhip_matmul_i8_dev stays bit-exact for every token count, and
+ * runs in its place where d_q is not 16-byte aligned. */
 int32_t nhip_matmul_i8_fused_dev(const nhip_weights* w, const int8_t* d_q, const float* d_qscale,
                                  int32_t tokens, float* d_y, int32_t ldy, int32_t row_start,
                                  int32_t row_end, void* stream);
 
 /* Scalar.MatMulRows on device for codebook weights (Scalar.cs:146-192):
- * activations as produced by nhip_prepare_dev. */
+ * activations as produced by nhip_prepare_dev (d_values' alignment as
+ * nhip_matmul_i8_dev's d_q). */
 int32_t nhip_matmul_cq_dev(const nhip_weights* w, const int8_t* d_values, const float* d_scales,
                            const float* d_offsets, int32_t stride, int32_t tokens, float* d_y,
                            int32_t ldy, int32_t row_start, int32_t row_end, void* stream);

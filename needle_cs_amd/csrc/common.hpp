@@ -100,6 +100,8 @@ struct nhip_weights : nhip::DeviceWeights {};
 namespace nhip {
 // Prefill matmul of the literal int8 format (gemm.hip): exact = Scalar
 // order (bit-identical with the decode kernels), else the fused epilogue.
+// 1 without launching when q is not 16-byte aligned (its copies into LDS are
+// 16 bytes): the general kernel takes such a call, in Scalar's order.
 int32_t launch_gemm_i8(const DeviceWeights* w, const int8_t* q, const float* qscale, int32_t tokens, float* y,
                        int32_t ldy, int32_t row_start, int32_t row_end, bool exact, hipStream_t stream);
 // Prefill matmul of the codebook formats (gemm_cq.hip), more than 16 tokens:

@@ -279,6 +279,7 @@ int32_t launch(const GemmParams& p, bool special, hipStream_t stream)
 int32_t launch_gemm_i8(const DeviceWeights* w, const int8_t* q, const float* qscale, int32_t tokens, float* y,
                        int32_t ldy, int32_t row_start, int32_t row_end, bool exact, hipStream_t stream)
 {
+    if (reinterpret_cast<uintptr_t>(q) & 15) return 1;  // (16-byte copies into LDS; K is a multiple of 32)
     GemmParams p{};
     p.tiles = w->tiles;
     p.norms = w->norms;
@@ -316,5 +317,7 @@ extern "C" int32_t nhip_matmul_i8_fused_dev(const nhip_weights* w, const int8_t*
     NHIP_REQUIRE(d_q && d_qscale && d_y, "null pointer");
     int32_t rc = ensure_device();
     if (rc) return rc;
-    return launch_gemm_i8(w, d_q, d_qscale, tokens, d_y, ldy, row_start, row_end, false, as_stream(stream));
+    rc = launch_gemm_i8(w, d_q, d_qscale, tokens, d_y, ldy, row_start, row_end, false, as_stream(stream));
+    if (rc <= 0) return rc;
+    return nhip_matmul_i8_dev(w, d_q, d_qscale, tokens, d_y, ldy, row_start, row_end, stream);
 }

@@ -1812,8 +1812,10 @@ int32_t run_matmul(const DeviceWeights* w, const int8_t* q, const float* scales,
         return launch_gemm_cq(w->format, t, w->special_scales != 0, stream);
     }
     if (w->format == WeightFormat::Int8G32) {
-        if (!dots && tokens >= kGemmMinTokens)
-            return launch_gemm_i8(w, q, scales, tokens, y, ldy, row_start, row_end, true, stream);
+        if (!dots && tokens >= kGemmMinTokens) {
+            const int32_t grc = launch_gemm_i8(w, q, scales, tokens, y, ldy, row_start, row_end, true, stream);
+            if (grc <= 0) return grc;
+        }
         if (!dots) {
             const int32_t nrc = launch_i8_narrow(w, 0, q, nullptr, nullptr, scales, 0.0f, nullptr, tokens, y, ldy,
                                                  row_start, row_end, stream);

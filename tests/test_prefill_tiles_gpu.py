@@ -89,3 +89,22 @@ def test_int8_tiles_bit_exact(hip, orc, tokens, rows, cols):
     # stated bound
     yf = run_fused(hip, weights, q, qs, tokens, rows, 0, rows)
     assert np.max(np.abs(yf.astype(np.float64) - want)) <= 1e-4 * float(np.sqrt(np.mean(want.astype(np.float64) ** 2)))
+
+
+@pytest.mark.parametrize("shift", [4, 8])
+@pytest.mark.parametrize("tokens,rows,cols", [(3, 64, 1024), (17, 70, 96), (31, 100, 288), (64, 130, 256), (200, 48, 2048)])
+def test_int8_activations_off_16_bytes(hip, orc, tokens, rows, cols, shift):
+    """Activations 4 or 8 bytes past a 16-byte boundary: both entries run in
+    the reference's order, in the kernels that load them through registers."""
+    w, scales, x, q, qs = int8_case(orc, tokens + rows + shift, rows, cols, tokens)
+    weights = hip.Weights.int8(w, scales)
+    want = np.full((tokens, rows), SENTINEL, dtype=np.float32)
+    orc.matmul_rows_i8(w, scales, q, qs, tokens, want, rows, 0, rows)
+    v = np.zeros(tokens * cols + shift, dtype=np.int8)
+    v[shift:] = q.reshape(-1)
+    dq, ds = hip.DeviceBuffer.from_array(v), hip.DeviceBuffer.from_array(qs)
+    lib = hip.lib()
+    for entry in (lib.nhip_matmul_i8_dev, lib.nhip_matmul_i8_fused_dev):
+        dy = hip.DeviceBuffer.from_array(np.full(tokens * rows, SENTINEL, dtype=np.float32))
+        hip.check(entry(weights.handle, dq.ptr + shift, ds.ptr, tokens, dy.ptr, rows, 0, rows, None))
+        assert np.array_equal(dy.download(np.float32).view(np.uint32), want.reshape(-1).view(np.uint32))
