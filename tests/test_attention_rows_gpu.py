@@ -1,7 +1,7 @@
-"""Attention of many rows (the group kernel of attention_decode.hip): bit-exact
-with the oracle's chunk-and-merge restatement over the group sizes, workgroup
-sizes, chunk counts and span lengths at which its launch and its rounds change;
-invalid spans give zeros."""
+"""Attention of many rows: bit-exact with the oracle's chunk-and-merge
+restatement on both sides of the group kernel's dispatch (attention_decode.hip),
+in each of its forms (workgroup threads, heads a thread), over chunk counts and
+span lengths at which its rounds change; invalid spans give zeros."""
 import numpy as np
 import pytest
 
@@ -39,5 +39,36 @@ def test_many_rows_short_caches_and_invalid_spans(hip, orc, heads, kv_heads, cap
     got, _ = run_decode(hip, cache, q, qs, heads, spec, 8)
     good = [k for k in range(rows) if k not in bad]
     want = oracle_decode(orc, cache, q, qs, heads, [spec[k] if k not in bad else (0, 0, 0) for k in range(rows)], 8)
+    assert bit_equal(got[good], want[good])
+    assert np.all(got[list(bad)] == 0.0)
+
+
+# the group kernel's forms, (threads, heads a thread)
+FORMS = [
+    ((256, 1), 4, 4, 64, 100, 600, 16), ((256, 1), 16, 8, 64, 140, 500, 8), ((256, 2), 32, 8, 64, 66, 300, 8),
+    ((256, 3), 12, 2, 48, 300, 300, 8), ((512, 1), 8, 8, 64, 100, 1000, 64), ((512, 1), 8, 4, 48, 70, 800, 16),
+    ((512, 2), 12, 2, 48, 400, 500, 8), ((512, 2), 4, 2, 64, 200, 2300, 64), ((512, 3), 12, 4, 48, 65, 700, 32),
+    ((512, 3), 12, 2, 64, 300, 1000, 64), ((1024, 1), 5, 1, 64, 66, 1024, 64), ((1024, 1), 12, 2, 48, 100, 2048, 8),
+    ((1024, 2), 4, 1, 48, 70, 530, 64), ((1024, 2), 16, 1, 64, 100, 600, 8), ((1024, 3), 12, 2, 64, 70, 1020, 64),
+]
+
+
+@pytest.mark.parametrize("form,heads,kv_heads,qk,rows,capacity,max_chunks", FORMS)
+def test_group_forms_bit_exact(hip, orc, form, heads, kv_heads, qk, rows, capacity, max_chunks):
+    cache = Cache(orc, hip, sum(form) + heads + capacity, 2, capacity, kv_heads, qk)
+    rng = np.random.default_rng(rows + capacity + heads)
+    edge = [1, 2, 16, 17, 31, 33, 48, capacity // 2 + 1, capacity - 1, capacity]
+    spec = [(k % 2, 0, c) for k, c in enumerate(edge)] + [(1, 5, 40), (0, capacity - 1, 1), (1, capacity - 33, 33)]
+    while len(spec) < rows:
+        first = int(rng.integers(0, capacity))
+        spec.append((int(rng.integers(0, 2)), first, int(rng.integers(1, capacity - first + 1))))
+    bad = {20: (2, 0, 10), 21: (1, -1, 5), 40: (0, 0, 0), 41: (1, capacity - 10, 25), rows - 1: (-1, 0, 3)}
+    for k, v in bad.items():
+        spec[k] = v
+    q, qs = queries(orc, cache.st, rows, heads, qk)
+    got, _ = run_decode(hip, cache, q, qs, heads, spec, max_chunks)
+    good = [k for k in range(rows) if k not in bad]
+    want = oracle_decode(orc, cache, q, qs, heads, [spec[k] if k not in bad else (0, 0, 0) for k in range(rows)],
+                         max_chunks)
     assert bit_equal(got[good], want[good])
     assert np.all(got[list(bad)] == 0.0)

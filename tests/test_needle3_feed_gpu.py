@@ -1,7 +1,8 @@
 """FeedSlot's long steps: a prompt longer than the context's chunk reaches the
-bits of the same prompt fed chunk by chunk, over the edges of a step (512 rows)
-and of the context, with a decode step after it; and a token out of range
-leaves what the chunk-by-chunk feed leaves."""
+bits of the same prompt fed chunk by chunk, over the edges of a step (512 rows,
+after a history of 3), in several steps and at the context's end, with decode
+steps after it; feeds of a captured step's rows between decode steps; and a
+token out of range leaves what the chunk-by-chunk feed leaves."""
 import numpy as np
 import pytest
 
@@ -10,7 +11,8 @@ from test_needle3_step_gpu import archive, gpu_engine, model, same_bits, tokens 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("count,capacity", [(17, 64), (130, 160), (512, 560), (513, 560), (90, 91)])
+@pytest.mark.parametrize("count,capacity", [(17, 64), (130, 160), (512, 560), (513, 560), (90, 91),
+                                            (515, 560), (516, 560), (1100, 1150)])
 def test_long_feed_equals_chunks(hip, model, count, capacity):  # noqa: F811
     p = tokens(1000 + count, count)
     a = gpu_engine(model, slots=2, capacity=capacity, chunk=16)
@@ -27,6 +29,28 @@ def test_long_feed_equals_chunks(hip, model, count, capacity):  # noqa: F811
         assert a.slot_length(1) == count
         for t in tokens(7, min(3, capacity - count)):
             assert same_bits(a.forward_batch([t], [1], [0])[0], b.forward_batch([t], [1], [0])[0])
+    finally:
+        a.close()
+        b.close()
+
+
+def test_short_feeds_between_decode_steps(hip, model):  # noqa: F811
+    """A chunk of 4: feeds of 10 rows are one captured step over the long steps'
+    inputs, replayed between decode steps over the short ones'."""
+    a = gpu_engine(model, slots=3, capacity=96, chunk=4)
+    b = gpu_engine(model, slots=3, capacity=96, chunk=4)
+    try:
+        for rep in range(4):
+            for slot in (0, 2):
+                p = tokens(60 + 3 * rep + slot, 10)
+                got = a.feed_slot(slot, p)
+                for start in range(0, 10, 4):
+                    n = min(4, 10 - start)
+                    last = start + n == 10
+                    want = b.forward_batch(p[start:start + n], [slot] * n, [n - 1] if last else [])[0]
+                assert same_bits(got, want[0]), (rep, slot)
+            t = tokens(90 + rep, 3)
+            assert same_bits(a.forward_batch(t, [0, 1, 2], [0, 1, 2])[0], b.forward_batch(t, [0, 1, 2], [0, 1, 2])[0]), rep
     finally:
         a.close()
         b.close()
