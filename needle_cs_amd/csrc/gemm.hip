@@ -54,6 +54,7 @@ struct GemmParams {
     float* y;
     int32_t tokens, cols, groups, blocks, groups_pad8, ldy;
     int32_t row_start, row_end, tile_begin, tile_end;
+    uint32_t row_blocks, token_blocks;  // the grid
 };
 
 template <int TPW>
@@ -64,7 +65,8 @@ struct WStage {
 
 // Four waves per workgroup, each owning TPW 16-row tiles (at 64 tokens two
 // tiles a wave measured fastest: one reads the A operands twice as often).
-template <bool EXACT, bool SPECIAL, int TI, int TPW>
+// RENUMBER: the workgroups by XCD (launch_tile).
+template <bool EXACT, bool SPECIAL, int TI, int TPW, bool RENUMBER>
 __device__ __forceinline__ void gemm_i8_body(const GemmParams& p)
 {
     constexpr int WAVES = 4;
@@ -76,8 +78,15 @@ __device__ __forceinline__ void gemm_i8_body(const GemmParams& p)
     const int wave = tid >> 6;
     const int r = lane & 15;
     const int kq = lane >> 4;
-    const int t0 = blockIdx.y * (16 * TI);
-    const int tile0 = p.tile_begin + blockIdx.x * (WAVES * TPW) + wave * TPW;
+    int bx = blockIdx.x, by = blockIdx.y;
+    if constexpr (RENUMBER) {
+        const uint32_t id = by * p.row_blocks + bx, total = p.row_blocks * p.token_blocks, xcd = id & 7;
+        const uint32_t block = xcd * (total >> 3) + min(xcd, total & 7) + (id >> 3);
+        bx = block / p.token_blocks;
+        by = block - bx * p.token_blocks;
+    }
+    const int t0 = by * (16 * TI);
+    const int tile0 = p.tile_begin + bx * (WAVES * TPW) + wave * TPW;
     const int stages = (p.blocks + kStage - 1) / kStage;
 
     const u4* wbase[TPW];
@@ -236,23 +245,41 @@ __device__ __forceinline__ void gemm_i8_body(const GemmParams& p)
     }
 }
 
-template <bool EXACT, bool SPECIAL, int TI, int TPW>
+template <bool EXACT, bool SPECIAL, int TI, int TPW, bool RENUMBER>
 __global__ __launch_bounds__(256) void gemm_i8_kernel(GemmParams p)
 {
-    gemm_i8_body<EXACT, SPECIAL, TI, TPW>(p);
+    gemm_i8_body<EXACT, SPECIAL, TI, TPW, RENUMBER>(p);
+}
+
+template <bool EXACT, int TI, int TPW, bool RENUMBER>
+int32_t launch_kernel(const GemmParams& p, bool special, hipStream_t stream)
+{
+    const dim3 grid(p.row_blocks, p.token_blocks);
+    if (special)
+        hipLaunchKernelGGL((gemm_i8_kernel<EXACT, true, TI, TPW, RENUMBER>), grid, dim3(256), 0, stream, p);
+    else
+        hipLaunchKernelGGL((gemm_i8_kernel<EXACT, false, TI, TPW, RENUMBER>), grid, dim3(256), 0, stream, p);
+    NHIP_CHECK_HIP(hipGetLastError());
+    return NHIP_OK;
 }
 
 template <bool EXACT, int TI, int TPW>
-int32_t launch_tile(const GemmParams& p, bool special, hipStream_t stream)
+int32_t launch_tile(GemmParams p, bool special, hipStream_t stream)
 {
     const int tiles = p.tile_end - p.tile_begin;
-    dim3 grid((tiles + 4 * TPW - 1) / (4 * TPW), (p.tokens + 16 * TI - 1) / (16 * TI));
-    if (special)
-        hipLaunchKernelGGL((gemm_i8_kernel<EXACT, true, TI, TPW>), grid, dim3(256), 0, stream, p);
-    else
-        hipLaunchKernelGGL((gemm_i8_kernel<EXACT, false, TI, TPW>), grid, dim3(256), 0, stream, p);
-    NHIP_CHECK_HIP(hipGetLastError());
-    return NHIP_OK;
+    p.row_blocks = (tiles + 4 * TPW - 1) / (4 * TPW);
+    p.token_blocks = (p.tokens + 16 * TI - 1) / (16 * TI);
+    // Workgroups go to the 8 XCDs in turn, so a row block's token blocks share
+    // one XCD's L2 only if the row blocks are a multiple of 8.  Otherwise the
+    // kernel renumbers them (a permutation): XCD c's, in order, take the c-th
+    // eighth of the blocks, a row block's token blocks one after another.  Fused
+    // 700 x 4096 x 5001 in 79 row blocks of 64: 74.9 -> 54.8 us; exact 130 x
+    // 2048 x 5000: 16.0 -> 11.4.  With less than 16 MB of weight blocks read again
+    // it gains nothing (24 x 1056 x 5000 4.3 us) and its division costs 0.1 us.
+    const bool renumber =
+        p.row_blocks % 8 != 0 && (int64_t)tiles * p.blocks * (p.token_blocks - 1) >= 16384;  // (blocks of 1 KB)
+    return renumber ? launch_kernel<EXACT, TI, TPW, true>(p, special, stream)
+                    : launch_kernel<EXACT, TI, TPW, false>(p, special, stream);
 }
 
 template <bool EXACT>
@@ -262,15 +289,18 @@ int32_t launch(const GemmParams& p, bool special, hipStream_t stream)
     const auto groups_of = [&](int ti, int tpw) {  // workgroups of a launch
         return (int64_t)((tiles + 4 * tpw - 1) / (4 * tpw)) * ((p.tokens + 16 * ti - 1) / (16 * ti));
     };
-    // The largest tile that leaves two workgroups for every CU.  Measured for
-    // 64 x 128 / 32 x 64 / 16 x 64, exact (before the two register sets):
-    // 512 x 2048 x 8192 38.7 / 41.8 / - us (512 workgroups of 64 x 128);
-    // 512 x 2048 x 4096 27.2 / 22.8 / 28.3 (256); 128 x 1024 x 8192 14.4 / 8.1 /
-    // 8.6 (128; 512 of 32 x 64); 256 x 1024 x 3072 14.2 / 7.7 / 7.2 (384 of
-    // 32 x 64); 128 x 1024 x 1024 13.5 / 5.6 / 4.2; 128 x 4096 x 1024 43.7 /
-    // 15.6 / 11.5 (one chain of 128 groups a wave).
-    if (groups_of(4, 2) >= 512) return launch_tile<EXACT, 4, 2>(p, special, stream);
-    if (groups_of(2, 1) >= 512) return launch_tile<EXACT, 2, 1>(p, special, stream);
+    // The largest tile that leaves about two workgroups for every CU; in the
+    // fused form, whose epilogue is shorter, the larger ones pay sooner (32 x 64
+    // from K 2048; below, 16 x 64 is 1% to 2% faster there).
+    // Measured, 64 x 128 / 32 x 64 / 16 x 64:
+    //   exact 512 x 2048 x 8192 (512 workgroups of 64 x 128) 39.7 / 40.5 / 50.9 us;
+    //   459 x 2048 x 7540 (472) 38.2 / 36.2 / 45.6; 200 x 2048 x 4000 (441 of
+    //   32 x 64) 22.5 / 12.4 / 14.2; 130 x 2048 x 5000 (395) 22.4 / 11.8 / 11.3
+    //   fused 512 x 2048 x 7168 (448) 28.2 / 30.4 / 43.4; 1000 x 1024 x 3000 (384)
+    //   16.6 / 15.2 / 20.0; 128 x 2048 x 4096 (256 of 32 x 64) 15.7 / 7.0 / 7.5;
+    //   128 x 2048 x 2048 (128) 15.6 / 6.5 / 5.8
+    if (groups_of(4, 2) >= (EXACT ? 512 : 400)) return launch_tile<EXACT, 4, 2>(p, special, stream);
+    if (groups_of(2, 1) >= (EXACT || p.blocks < 32 ? 420 : 256)) return launch_tile<EXACT, 2, 1>(p, special, stream);
     return launch_tile<EXACT, 1, 1>(p, special, stream);
 }
 

@@ -77,6 +77,8 @@ def test_codebook_batch_jobs_end_inside_a_tile(hip, orc, bits, tokens, rows):
     (20, 70, 288),      # a partial last stage
     (250, 4099, 96),    # 32 x 64
     (1000, 4090, 288),  # 64 x 128
+    # row blocks not a multiple of 8, renumbered over the XCDs: each tile
+    (33, 2300, 4096), (250, 4099, 608), (1000, 4500, 480),
 ])
 def test_int8_tiles_bit_exact(hip, orc, tokens, rows, cols):
     w, scales, x, q, qs = int8_case(orc, tokens + rows, rows, cols, tokens)
