@@ -1779,11 +1779,12 @@ int32_t launch_group_hpt(const DecodeAttnParams& p, int hpt, size_t lds, hipStre
 //  - few (row, chunk) workgroups: 44 rows, 12 heads on 2, up to 1024 positions in
 //    64 chunks 15.5 and 18.6, 54 rows 17.9 and 18.3, 128 rows 45.3 and 19.7
 //  - spans the whole-row kernel takes (512 positions): its workgroups, one per
-//    (row, head), are enough up to about 1344 of them (12 on 2, 88 rows of up to
-//    176 8.9 and 10.3, 128 rows of up to 256 12.8 and 11.6), and with two heads a
-//    group up to 2048 and past 16 chunks (16 on 8, 66 rows 12.4 and 13.3; 300
-//    rows 41.8 and 32.5, but in 64 chunks 20.6 and 29.9 when they are short);
-//    large groups need a workgroup for every CU (16 on 1, 66 rows 15.1 and 20.2)
+//    (row, head), are enough up to about 1344 of them unless the spans are long
+//    (12 on 2, 88 rows of up to 176 8.9 and 10.3, 128 rows of up to 256 12.8 and
+//    11.6, 87 rows up to 437 16.6 and 12.8), and with two heads a group up to 2048
+//    and past 16 chunks (16 on 8, 66 rows 12.4 and 13.3; 300 rows 41.8 and 32.5,
+//    but in 64 chunks 20.6 and 29.9 when they are short); large groups need a
+//    workgroup for every CU (16 on 1, 66 rows 15.1 and 20.2)
 //  - one head a group shares nothing, so what there is to gain is the empty
 //    chunks and the merge: 8 on 8, 100 rows of up to 1024 in 8 chunks 23.2 and
 //    29.0, in 64 27.1 and 27.9 (growing spans 21.9 and 12.6); 66 rows in 64
@@ -1791,45 +1792,51 @@ int32_t launch_group_hpt(const DecodeAttnParams& p, int hpt, size_t lds, hipStre
 //  - rows over caches of their own, which only the chunk kernel reads in whole
 //    cache rows: 96 rows, 16 heads on 8, 2048 positions 38.6 and 55.7 (100 rows, 12
 //    on 2, 1024 positions 26.5 and 17.8)
-//  - past 1024 positions the longest rows set the time unless the workgroups are
-//    about one a CU, or many and the chunks too: 4 on 1, 66 rows of up to 2048 in
-//    16 chunks 18.4 and 25.8; 12 on 2, 100 rows in 8 38.3 and 36.0, 160 rows 45.7
-//    and 62.0; 8 on 4, 160 rows in 64 45.0 and 43.2 (growing spans 27.2 and 14.2),
-//    16 on 8 58.5 and 77.0; of up to 4096 8 on 4 61.4 and 87.5, 4 on 2, 256 rows
-//    66.0 and 65.8 (growing spans 38.2 and 16.2)
+//  - past 1024 positions a row's length shows.  Up to a workgroup a CU that many
+//    CUs idle for it: 4 on 1, 48 rows of 1760 14.7 and 21.4, 128 rows of 2142 36.9
+//    and 25.1; 8 on 4, 57 rows of 3616 40.5 and 31.2.  Beyond, a CU with one
+//    workgroup more than the others sets the time: 16 on 4, 68 rows of 1963 39.2
+//    and 53.9, 186 rows of 3385 55.8 and 42.3; the chunks have to be many, 12 on 2,
+//    160 rows of up to 2048 in 8 chunks 45.7 and 62.0; and from 8 kv heads the
+//    chunk kernel's whole cache rows win again: 16 on 8, 104 rows of 1067 30.5 and
+//    21.3, 45 of 3149 40.6 and 60.5
 //  - few chunks and few workgroups of large groups (16 on 1, 66 rows of up to 600
 //    in 8 20.2 and 22.4), or few heads a group (12 on 4, 66 rows in 8 21.8 and
 //    28.3)
 // A batch with one row far longer than the rest can still take up to 1.3 times as
 // long here (128 rows of up to 40 positions and one of 2047, 8 on 4: 24.9 and
-// 31.3): its chunks run in one workgroup.
-bool takes_group(const DecodeAttnParams& p, int span, int chunks)
+// 31.3): its chunks run in one workgroup.  per_cu: workgroups a CU holds.
+bool takes_group(const DecodeAttnParams& p, int span, int chunks, int per_cu)
 {
     const int group = p.heads / p.kv_heads;
     const int64_t blocks = (int64_t)p.rows * p.kv_heads;
     const bool own = p.rows < 8 * (int64_t)p.slots;  // few rows a slot
-    if (p.rows <= kPlacedRows && p.rows * chunks <= 3072) return false;
+    const bool wide = p.kv_heads >= 8;
+    if (p.rows <= kPlacedRows && p.rows * chunks <= (blocks < 128 || (wide && group <= 2) ? 3072 : 2560)) return false;
     if (own && (group == 1 || span > 1024 || blocks > 1024)) return false;
     if (span <= kRowMaxCapacity) {
         if (group == 1 || (group > 8 && blocks <= p.cus)) return false;
-        return group == 2 ? chunks <= 16 && blocks >= 1024 : blocks * group >= 1344;
+        if (group == 2) return chunks <= 16 && blocks >= 1024;
+        return blocks * group >= 1344 || (p.kv_heads > 1 && blocks * group * span >= 450000);
     }
     if (group == 1)
         return span <= 1024 && p.kv_heads <= 8 && chunks >= 4 * p.kv_heads &&
-               (p.rows >= 96 || chunks >= 16 * p.kv_heads);
-    if (span > 1024) {
-        if (span <= 2048 && blocks <= p.cus && 2 * blocks >= p.cus) return true;
-        return p.rows >= 96 && 2 * blocks >= 3 * p.cus && chunks >= 12 * p.kv_heads &&
-               (span <= 2048 || p.kv_heads <= 2);
+               (p.rows >= 96 || chunks > 8 * p.kv_heads);
+    if (span <= 1024) {
+        if (group > 4 && blocks < 96 && chunks < 16) return false;
+        return chunks >= 4 * p.kv_heads || (group % 2 == 0 && (group > 2 || p.kv_heads <= 4));
     }
-    if (group > 4 && blocks < 96 && chunks < 16) return false;
-    return chunks >= 4 * p.kv_heads || (group % 2 == 0 && (group > 2 || p.kv_heads <= 4));
+    if (blocks <= p.cus) return blocks * (group > 2 ? 22 : 33) >= span && (2 * blocks >= p.cus || chunks >= 32);
+    const int64_t most = (blocks + p.cus - 1) / p.cus;  // workgroups of the busiest CU
+    const float busy = (float)blocks / (float)(most * p.cus);
+    if (wide) return span <= 1500 && chunks >= 32 && busy >= 0.7f;
+    return chunks >= 12 * p.kv_heads && busy >= (per_cu > 1 || span <= 2048 ? 0.55f : 0.9f);
 }
 
 // The group kernel for batches of many rows whose spans are at most max_count
 // positions (0: unknown, up to the capacity); 1 when it does not take them
-// (takes_group, or an LDS layout past the CU's; where LDS leaves one workgroup a
-// CU, more than three rounds of them).
+// (takes_group), its LDS layout passes the CU's, or the workgroups would run in
+// more than four rounds (three of one workgroup a CU).
 // T: 1024 threads while every workgroup has a CU of its own (128 rows of up to
 // 1024, 12 on 2, 64 chunks: 19.7 us, 512 threads 24.3), then 512, or 256 for
 // short spans and few chunks (300 rows of up to 300, 8 chunks: 14.5 us, 512
@@ -1841,7 +1848,6 @@ int32_t launch_group_attention(DecodeAttnParams p, int32_t max_count, hipStream_
     const int group = p.heads / p.kv_heads;
     const int span = span_bound(max_count, p.capacity);
     const int chunks = std::min(p.max_chunks, std::max(span / 16, 1));
-    if (!takes_group(p, span, chunks)) return 1;
     const int64_t blocks = (int64_t)p.rows * p.kv_heads;
     const int T = blocks <= p.cus ? 1024 : span > 384 && chunks * 16 * group >= 512 ? 512 : 256;
     const auto fills = [&](int hpt, float share) {
@@ -1851,6 +1857,7 @@ int32_t launch_group_attention(DecodeAttnParams p, int32_t max_count, hipStream_
     const size_t lds = group_lds(span, p.max_chunks, T, group, hpt);
     if (lds > (size_t)kGroupMaxLds) return 1;
     const int per_cu = std::min(2048 / T, (int)(kGroupMaxLds / lds));
+    if (!takes_group(p, span, chunks, per_cu)) return 1;
     if (blocks > (int64_t)(per_cu > 1 ? 4 : 3) * p.cus * per_cu) return 1;
     p.lmax = span;
     return T == 1024 ? launch_group_hpt<1024>(p, hpt, lds, stream)
