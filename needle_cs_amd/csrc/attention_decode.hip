@@ -1183,8 +1183,11 @@ __global__ __launch_bounds__(row_threads(MODE)) void decode_attention_row_kernel
         }
     }
     float* dst = p.out + ((size_t)row * p.heads + h) * 64;
+    // (in the plain form no count passes kRowMaxCapacity: the capacity does not,
+    // or the engine that passed max_count wrote the counts; that comparison on
+    // the way to the first loads took 0.1 to 0.2 us of 5.8)
     const bool valid = (slot_in >= 0) & (slot_in < p.slots) & (first_in >= 0) & (count_in >= 1) &
-                       (count_in <= p.capacity - first_in) & (count_in <= kRowMaxCapacity);
+                       (count_in <= p.capacity - first_in) & (MODE == kRowPlain || count_in <= kRowMaxCapacity);
     const int slot = valid ? slot_in : 0;
     const int first = valid ? first_in : 0;
     const int count = valid ? count_in : 1;
@@ -1204,7 +1207,7 @@ __global__ __launch_bounds__(row_threads(MODE)) void decode_attention_row_kernel
         }
     }
     int length;
-    const int needed = plan(count, p.max_chunks, &length);  // count <= capacity <= 512: needed <= 32
+    const int needed = plan(count, p.max_chunks, &length);  // count <= 512: needed <= 32
     const uint32_t mag_len = magic((uint32_t)length);       // s < 512: s / length is exact
     const size_t pos0 = (size_t)slot * p.capacity + first;
     const int qk = p.qk;
