@@ -528,7 +528,9 @@ int32_t nhip_model_close(nhip_model* m);
  * independent sequences of up to `capacity` positions each, steps of up to
  * `chunk` rows (0: the reference's default 64).  Attention splits a row's
  * span into at most `max_chunks` chunks by the reference's plan (0: 8, the
- * reference's MaxChunks, Blocks.cs:832).  The model must stay open while the
+ * reference's MaxChunks, Blocks.cs:832).  Scratch is held for nhip_slot_feed's
+ * long steps too, min(512, capacity) rows whatever the chunk (about 55 MB at
+ * Needle 3's geometry).  The model must stay open while the
  * context lives.  One context is single-threaded; it owns a HIP stream and
  * its device state (KV cache, convolution and engram histories, snapshots). */
 typedef struct nhip_ctx nhip_ctx;

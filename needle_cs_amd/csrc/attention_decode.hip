@@ -615,9 +615,10 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(ATTN_HEAD_PARAMS, Deco
 // What bounds it: the value walk's VALU work, a multiply and an add per
 // (position, head, dim) and 1 / HPT of the conversions (half of the time of
 // 128 rows of 1024 positions), and the latencies of the phases before it.
-// Measured, with the launch it replaces (and its merge): 128 rows of up to 1024
-// positions, 12 heads on 2, up to 64 chunks 19.7 us (45.3); 300 rows of up to
-// 300, 8 chunks 14.5 (25.8); 2 x 128 rows, 8 heads on 8, 64 chunks 43.0 (57.6).
+// Measured back to back in a graph, with the launch it replaces (and its merge):
+// 128 rows of up to 1024 positions, 12 heads on 2, up to 64 chunks 19.9 us (45.5);
+// 300 rows of up to 300, 8 chunks 15.0 (25.0); 2 x 128 rows, 8 heads on 8, 64
+// chunks 45 (58.7).
 constexpr int kGroupMaxLds = 160 * 1024;
 constexpr int group_chunks_per_round(int T, int group, int hpt) { return T / (16 * ((group + hpt - 1) / hpt)); }
 constexpr int group_row_ld(int capacity) { return ((capacity + 15) & ~15) + 4; }
@@ -1780,7 +1781,7 @@ int32_t launch_group_hpt(const DecodeAttnParams& p, int hpt, size_t lds, hipStre
 // batches of 40 to 900 rows, timed both ways with short, growing, middling,
 // random and long spans.  Microseconds, the other kernels first and then this:
 //  - few (row, chunk) workgroups: 44 rows, 12 heads on 2, up to 1024 positions in
-//    64 chunks 15.5 and 18.6, 54 rows 17.9 and 18.3, 128 rows 45.3 and 19.7
+//    64 chunks 15.5 and 18.6, 54 rows 17.9 and 18.3, 128 rows 45.5 and 19.9
 //  - spans the whole-row kernel takes (512 positions): its workgroups, one per
 //    (row, head), are enough up to about 1344 of them unless the spans are long
 //    (12 on 2, 88 rows of up to 176 8.9 and 10.3, 128 rows of up to 256 12.8 and
@@ -1841,9 +1842,9 @@ bool takes_group(const DecodeAttnParams& p, int span, int chunks, int per_cu)
 // (takes_group), its LDS layout passes the CU's, or the workgroups would run in
 // more than four rounds (three of one workgroup a CU).
 // T: 1024 threads while every workgroup has a CU of its own (128 rows of up to
-// 1024, 12 on 2, 64 chunks: 19.7 us, 512 threads 24.3), then 512, or 256 for
-// short spans and few chunks (300 rows of up to 300, 8 chunks: 14.5 us, 512
-// threads 15.8).  HPT: the most heads a thread that keep the threads busy (300
+// 1024, 12 on 2, 64 chunks: 512 threads take 4.6 us more), then 512, or 256 for
+// short spans and few chunks (300 rows of up to 300, 8 chunks: 512 threads take
+// 1.3 us more).  HPT: the most heads a thread that keep the threads busy (300
 // rows of up to 1024 in 8 chunks, 512 threads: 2 heads 40 us with 3/4 of them,
 // 3 heads 54 with half, 1 head 52).
 int32_t launch_group_attention(DecodeAttnParams p, int32_t max_count, hipStream_t stream)

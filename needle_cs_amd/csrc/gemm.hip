@@ -104,8 +104,8 @@ __device__ __forceinline__ void gemm_i8_body(const GemmParams& p)
         for (int e = 0; e < 4; e++) qs[i][e] = p.qscale[min(t0 + 16 * i + 4 * kq + e, p.tokens - 1)];
 
     // Activation staging, straight from memory into LDS (global_load_lds,
-    // no registers): per stage 32 blocks (group gs of the stage, 16-token
-    // subtile i) of 512 bytes, block b = 4*gs + i.  Position x (0..31) of a
+    // no registers): per stage 8 * TI blocks (group gs of the stage, 16-token
+    // subtile i) of 512 bytes, block b = TI * gs + i.  Position x (0..31) of a
     // block holds the 16 bytes of token 16i + x/2, k-slices 2p and 2p + 1 of
     // the group, with p = (x & 1) ^ bit 3 of the token ^ (i & 1): the MFMA
     // A reads (lane (t16, kq): 8 bytes at position 2*t16 + (kq/2 ^ ...),
@@ -146,7 +146,7 @@ __device__ __forceinline__ void gemm_i8_body(const GemmParams& p)
 #pragma unroll
             for (int e = 0; e < 4; e++) acc[j][i][e] = 0.0f;
 
-    // one stage: group k's A operands (four 16-token subtiles), its MFMAs
+    // one stage: group k's A operands (TI 16-token subtiles), its MFMAs
     // and its epilogue, software-pipelined so that group k+1's MFMAs and
     // group k+2's LDS reads are in flight during group k's epilogue
     auto read_a = [&](long (&av)[TI], int buf, int k) {

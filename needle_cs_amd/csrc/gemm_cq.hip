@@ -153,7 +153,7 @@ __device__ __forceinline__ void gemm_cq_body(const TileMatmul& p)
             for (int e = 0; e < 4; e++) acc[j][i][e] = bias[j][i][e] = 0.0f;
 
     auto group = [&](const WStage<CQ4, TPW>& x, int buf, int k) {
-        // the A operands of the four subtiles
+        // the A operands of the TI subtiles
         v4i a[TI][2];
 #pragma unroll
         for (int i = 0; i < TI; i++)
@@ -287,7 +287,8 @@ int32_t launch_form(const TileMatmul& p, bool special, hipStream_t s)
     const auto groups_of = [&](int ti, int tpw) {  // workgroups of a launch
         return (int64_t)((tiles + 4 * tpw - 1) / (4 * tpw)) * ((p.tokens + 16 * ti - 1) / (16 * ti));
     };
-    // The largest tile whose grid still covers the chip's 256 CUs.  64 x 128
+    // The largest tile whose grid gives three quarters of the 256 CUs a workgroup
+    // (64 x 128), or one and a half to each (32 x 64).  64 x 128
     // takes about as long for 128 workgroups as for 256 (19.5 us at K 2048) and
     // loses to four times as many of 32 x 64 at 128 (13.5 us); 32 x 64 and
     // 16 x 64 meet near 400 (Cq2 512 x 768 x 1568, 400: 6.7 against 6.8 us;

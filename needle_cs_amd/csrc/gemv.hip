@@ -1733,11 +1733,14 @@ bool plan_general_cq(const DeviceWeights* w, MatmulParams& p, int waves, size_t*
 
 // Whether gemm_cq.hip takes a codebook matmul of `tokens` rows over `tiles` row
 // tiles, or the general kernel, whose waves split the groups of a 16 x 16 block
-// while gemm_cq's run through all of them.  The general kernel takes about
-// 3.2 us (Cq4) or 6 us (Cq2, half as many waves busy per block) and 0.3 ns per
-// (block, group); gemm_cq 1.8 us and 0.42 us per group of its chain, and 0.1 ns.
-// Cq4 64 x 2048 x 2048: 5.5 us general, 8.6 here; 256 x 1024 x 2048: 8.3, 7.2;
-// Cq2 128 x 4096 x 768: 11.1, 13.5; 61 x 768 x 1568: 10.5, 4.3.
+// while gemm_cq's run through all of them.  Fitted over 350 shapes of 17 to 1024
+// tokens, the general kernel takes about 3.5 us and 0.4 ns per (block, group) in
+// Cq4, 7 us and 0.7 to 1.1 ns in Cq2 (half as many waves busy per block); gemm_cq
+// 2.8 us, 0.2 us per group of its chain and 0.14 ns.  The lines lie above where
+// those cross, so that no shape is slower than in the general kernel (at most
+// 1.03 times its time): Cq4 64 x 2048 x 2048 5.5 us general, 8.6 here; 256 x 1024 x
+// 2048 8.3, 7.2; 510 x 2432 x 897 24.9, 11.2; Cq2 128 x 4096 x 768 11.1, 13.5;
+// 61 x 768 x 1568 10.5, 4.3; 22 x 2048 x 3744 9.0, 7.2.
 bool takes_gemm_cq(WeightFormat fmt, int32_t groups, const int8_t* q, int32_t tokens, int32_t tiles)
 {
     if (tokens <= 16 || (reinterpret_cast<uintptr_t>(q) & 15)) return false;  // (16-byte copies into LDS)
@@ -1942,8 +1945,8 @@ int32_t launch_gen_batch_fmt(const MatmulBatch& b, int per, int waves, size_t ld
 
 // Quant.MatMulBatch.Run (src/Needle/Quant.cs:697-706, 753-772): every job's
 // MatMulRows over all its rows with the shared activations.  The decode
-// sizes (up to 16 tokens), and the codebook formats at any token count (the
-// general kernel), run as one launch over the row tiles of every job; the
+// sizes (up to 16 tokens), and the codebook formats at any token count
+// (gemm_cq.hip or the general kernel), run as one launch over the row tiles of every job; the
 // literal format past 16 tokens runs the jobs one after another (the same
 // kernels as nhip_matmul_*_dev, so the same bits either way).
 int32_t run_matmul_batch(const DeviceWeights* const* w, int32_t count, const int8_t* q, const float* scales,
