@@ -1,9 +1,8 @@
 """Writes tests/golden/needle3_golden.npz: the reference's own numpy forward
 of Needle 3 (tools/golden.py) on seeded random-init archives.
 
-Runs in the build container only (it imports the reference from
-/root/reference, which the GPU box does not have; .gpurunignore keeps this
-script off it).  Only the vectors it writes travel with the tests.
+Runs only where the reference's sources are at /root/reference, which it
+imports.  Only the vectors it writes travel with the tests.
 
 The reference holds its engine to this forward on the real model at cosine
 > 0.99995 with the same argmax (tests/Needle.Tests/ParityTests.cs:55-57).  Its
